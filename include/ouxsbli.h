@@ -220,7 +220,8 @@ int ox_kernel_times(ox_solver* s, ox_kernel_time* out, int32_t cap, int32_t* n);
 int ox_footprint(const ox_config* cfg, uint64_t* bytes);
 
 /* Picks the y- and z-sweep segment lengths for this handle's grid by timing
- * candidate values (16, 32, 64, 128 cells) on right-hand-side evaluations of
+ * the lengths in use (chosen by a rule on the grid at ox_create) and candidate
+ * values (16, 32, 64, 128 cells) on right-hand-side evaluations of
  * the current state, keeps the fastest in the handle and returns them.  The
  * state is not changed.  No reference counterpart (the reference's launch
  * shapes are fixed at build time, calc_flux_base.f90.fypp:44-63). */
@@ -229,8 +230,8 @@ int ox_autotune(ox_solver* s, int32_t* lseg_y, int32_t* lseg_z);
 /* Sets the y- and z-sweep segment lengths (cells one thread marches along the
  * sweep direction) explicitly, as ox_autotune would after timing them: any
  * value in 1..4096, lowered where the state offsets within one segment would
- * reach 2^31 ((lseg_z + 2) * 5 * nx * ny for z; for the default 64, planes of
- * over 6.5e6 cells).  Results do not depend on the choice; the setter exists so
+ * reach 2^31 ((lseg_z + 2) * 5 * nx * ny for z; for 64, planes of over 6.5e6
+ * cells).  Results do not depend on the choice; the setter exists so
  * that a caller can fix a tuned value, and a test can cover segment seams
  * deterministically.  No reference counterpart (fixed launch shapes,
  * calc_flux_base.f90.fypp:44-63). */

@@ -58,7 +58,8 @@ struct BCase {
   ox2d_solver* s2 = nullptr;
   int remaining;
   size_t bytes;
-  int group;  // index into ox_batch::groups while active
+  int group;    // index into ox_batch::groups while active
+  int solo[2];  // segment lengths of the case on its own (3-D)
 
   int dim() const { return s2 ? 2 : 3; }
   double cells() const {
@@ -196,6 +197,22 @@ int build_plan(ox_batch* b) {
     c->group = gi;
     b->groups[gi].members.push_back(c);
   }
+  // segment lengths: a case alone in its group keeps its own; cases that share
+  // launches get lengths for their tiles together, which fill the chip with
+  // longer segments than each would need by itself
+  for (BGroup& G : b->groups) {
+    if (G.dim == 2) continue;
+    for (int d = 1; d <= 2; ++d) {
+      std::vector<ox::LineWork> w;
+      for (BCase* c : G.members) w.push_back(ox::line_work(c->s->C.g, d));
+      const int together = ox::pick_lseg(w.data(), (int)w.size(), G.ops.line_occ(d), ox::device_cus());
+      for (size_t m = 0; m < w.size(); ++m) {
+        BCase* c = G.members[m];
+        c->s->C.lseg[d - 1] =
+            w.size() == 1 ? c->solo[d - 1] : ox::clamp_lseg(c->s->C.g, d, ox::even_lseg(w[m].cells, together));
+      }
+    }
+  }
   // tile maps: per 3-D group, per direction, one TileMap per member (LES
   // groups: three more, for the SGS viscosity and the two ghost-copy
   // passes); 2-D groups count their tiles (the case lookup reads the
@@ -222,9 +239,9 @@ int build_plan(ox_batch* b) {
         if (d == 0) {
           nbx = cdivu(g.ix, G.ops.xt); nby = cdivu(g.iy, ox::XROWS); nbz = g.iz;
         } else if (d == 1) {
-          nbx = cdivu(g.ix, ox::LINE_X); nby = cdivu(g.iz, ox::LINE_Y); nbz = cdivu(g.iy, ls[0]);
+          nbx = ox::line_tiles(g, 1); nby = 1; nbz = cdivu(g.iy, ls[0]);
         } else {
-          nbx = cdivu(g.ix, ox::LINE_X); nby = cdivu(g.iy, ox::LINE_Y); nbz = cdivu(g.iz, ls[1]);
+          nbx = ox::line_tiles(g, 2); nby = 1; nbz = cdivu(g.iz, ls[1]);
         }
         m.start = nt[d];
         m.nbx = (int)nbx;
@@ -499,6 +516,8 @@ int admit3d(ox_batch* b, const ox_config* cfg, Init init, int32_t nsteps, int64_
   c->remaining = nsteps;
   c->bytes = need;
   c->group = -1;
+  c->solo[0] = s->C.lseg[0];
+  c->solo[1] = s->C.lseg[1];
   b->bytes_in_use += need;
   *id = c->id;
   b->active.push_back(std::move(c));
@@ -539,16 +558,15 @@ int ox_autotune(ox_solver* s, int32_t* lseg_y, int32_t* lseg_z) {
     return ms;
   };
   static const int cand[] = {16, 32, 64, 128};
-  int by = ox::LSEG_DEFAULT, bz = ox::LSEG_DEFAULT;
-  float best = 1e30f;
+  int by = C.lseg[0], bz = C.lseg[1];  // the lengths in use, by rule unless set
+  float best = time_rhs(by, bz);
   for (int ly : cand) {
-    if (ly > 2 * g.iy && ly != cand[0]) continue;
+    if (ly > 2 * g.iy || ly == by) continue;
     const float t = time_rhs(ly, bz);
     if (t < best) best = t, by = ly;
   }
-  best = 1e30f;
   for (int lz : cand) {
-    if (lz > 2 * g.iz && lz != cand[0]) continue;
+    if (lz > 2 * g.iz || lz == bz) continue;
     const float t = time_rhs(by, lz);
     if (t < best) best = t, bz = lz;
   }

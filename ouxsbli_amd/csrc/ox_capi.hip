@@ -310,6 +310,21 @@ int run_rk_step(ox_solver* s) {
 }  // namespace
 
 namespace ox {
+int device_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 256;
+  return std::max(cus, 1);
+}
+
+void solo_segments(const Geom& g, const BatchOps& ops, int* lseg) {
+  for (int d = 1; d <= 2; ++d) {
+    const LineWork w = line_work(g, d);
+    lseg[d - 1] = clamp_lseg(g, d, even_lseg(w.cells, pick_lseg(&w, 1, ops.line_occ(d), device_cus())));
+  }
+}
+
 void launch_ghost_fill(Core& C, double* Q) {
   const Geom& g = C.g;
   const long long total = 2LL * g.h * g.nx * g.ny + (long long)g.iz * 2 * g.h * g.nx + (long long)g.iz * g.iy * 2 * g.h;
@@ -375,8 +390,7 @@ int ox_create(const ox_config* cfg, ox_solver** out) {
   C.prim_for = nullptr;
   C.prim_images[0] = C.prim_images[1] = false;
   C.stream = nullptr;
-  C.lseg[0] = ox::clamp_lseg(C.g, 1, ox::LSEG_DEFAULT);
-  C.lseg[1] = ox::clamp_lseg(C.g, 2, ox::LSEG_DEFAULT);
+  C.lseg[0] = C.lseg[1] = 1;  // set below, once the device is known
   C.prof = false;
   C.mark = &prof_record;
   C.prof_state = &s->prof;
@@ -391,7 +405,11 @@ int ox_create(const ox_config* cfg, ox_solver** out) {
   if (me4) C.vorder = 5;
   s->stage = cfg->precision == OX_PREC_FP64 ? ox::find_stage_fp64(cfg->order, cfg->scheme, cfg->visc, C.vorder)
                                             : ox::find_stage_fp32(cfg->order, cfg->scheme, cfg->visc, C.vorder);
-  if (!s->stage) {
+  ox::BatchOps ops;
+  const bool known = cfg->precision == OX_PREC_FP64
+                         ? ox::find_batch_fp64(cfg->order, cfg->scheme, cfg->visc, C.vorder, &ops)
+                         : ox::find_batch_fp32(cfg->order, cfg->scheme, cfg->visc, C.vorder, &ops);
+  if (!s->stage || !known) {
     delete s;
     return ox_fail(OX_EUNSUPPORTED, "no kernel specialisation for this (order, scheme, visc, visc_order)");
   }
@@ -400,6 +418,7 @@ int ox_create(const ox_config* cfg, ox_solver** out) {
     delete s;
     return ox_fail(OX_EDEVICE, std::string("hipSetDevice: ") + hipGetErrorString(e));
   }
+  ox::solo_segments(C.g, ops, C.lseg);
   const size_t ns = state_elems(C.g), nc = cell_elems(C.g);
   const size_t pe = cfg->precision == OX_PREC_FP64 ? sizeof(double) : sizeof(float);
   bool ok = hipStreamCreateWithFlags(&C.stream, hipStreamNonBlocking) == hipSuccess;

@@ -31,7 +31,7 @@ struct Core {
   // (FP64 in the plain form; FP32 in the FP32-bulk form, where it carries
   // FP32 flux differences and the RK combination itself stays FP64)
   void* Racc;
-  int lseg[2];       // segment lengths of the y and z sweeps (tuned per case)
+  int lseg[2];       // segment lengths of the y and z sweeps (by rule, tuned or set)
   hipStream_t stream;
   // profiling: when `prof` is set, mark() records an event after a kernel
   bool prof;
@@ -97,6 +97,8 @@ struct BatchOps {
   // the three sweep descriptors (x, y, z) of one case for one stage
   void (*make_args)(Core& C, const StageArgs& sa, double cx, double cy, double cz, void* out3);
   void (*launch)(const BatchGroupLaunch& L);
+  // workgroups of the line sweep along dir (1: y, 2: z) one compute unit holds
+  int (*line_occ)(int dir);
   // after a stage of one case with non-periodic directions: the ghost
   // primitives of the set its epilogue wrote (prims_new, 10 arrays), then the
   // Ducros sensors of the inner ghost layers
@@ -107,5 +109,10 @@ bool find_batch_fp64(int order, int scheme, int visc, int vorder, BatchOps* ops)
 bool find_batch_fp32(int order, int scheme, int visc, int vorder, BatchOps* ops);
 
 void launch_ghost_fill(Core& C, double* Q);
+
+// Compute units of the current device.
+int device_cus();
+// The y- and z-sweep segment lengths of a case that runs alone (pick_lseg).
+void solo_segments(const Geom& g, const BatchOps& ops, int* lseg);
 
 }  // namespace ox

@@ -496,15 +496,6 @@ __device__ __forceinline__ int xcd_tile(int b, int n) {
   return (b & 7) * (n >> 3) + (b >> 3);
 }
 
-// This workgroup's tile (bx, by, bz) of a 3-D launch under xcd_tile.
-__device__ __forceinline__ void launch_tile(int& bx, int& by, int& bz) {
-  const int gx = gridDim.x, gy = gridDim.y;
-  const int t = xcd_tile(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx * gy * gridDim.z);
-  bx = t % gx;
-  by = (t / gx) % gy;
-  bz = t / (gx * gy);
-}
-
 // The x sweep's tiles (bx, row band by, plane bz) in x, z, y order under
 // xcd_tile: one XCD's run covers a band of rows through many planes, so both
 // the y and the z neighbours a row tile's cross-derivative stencils read
@@ -971,15 +962,27 @@ __device__ __forceinline__ void fetch_state(const S* __restrict__ Racc, const St
 // R += c_y*(F_right - F_left); DIR=2 adds c_z*(G_right - G_left) and applies
 // the stage epilogue.
 // ---------------------------------------------------------------------------
-constexpr int LSEG_DEFAULT = 64;
-// Line-sweep workgroup: LINE_X consecutive x columns by LINE_Y rows (z rows
-// for the y sweep, y rows for the z sweep), 256 threads.
+// Line-sweep workgroup: LINE_X consecutive x cells by LINE_Y rows (y rows for
+// the z sweep, z rows for the y sweep), 256 threads.  The y sweep takes the
+// rows in groups of LINE_Y and runs through the cells of group after group, so
+// a workgroup whose x run reaches the end of the rows goes on in the next group
+// and only the last workgroup has idle lanes; with whole tiles 64 - ix % 64
+// lanes of every row's last tile idle (y sweep of the LES scheme at 96^3, FP64:
+// tiles 72 us, this 62 us; ME4 at 150 x 77 x 53: 60 and 57 us).  The z sweep, bound
+// by memory, keeps whole tiles: runs across rows slowed it (SLAU6 Euler at 124^3,
+// FP64: tiles 105 us, runs 111 us).
 #ifndef OX_LINE_X
 #define OX_LINE_X 64
 #endif
 constexpr int LINE_X = OX_LINE_X;
 constexpr int LINE_Y = 256 / LINE_X;
 static_assert(LINE_X % 64 == 0 && LINE_X * LINE_Y == 256, "line-sweep workgroup of whole wavefronts");
+// workgroups of one segment layer of the line sweep along dir
+__host__ __device__ inline unsigned line_tiles(const Geom& g, int dir) {
+  const long long groups = ((dir == 1 ? g.iz : g.iy) + LINE_Y - 1) / LINE_Y;
+  if (dir == 1) return (unsigned)((groups * g.ix + LINE_X - 1) / LINE_X);
+  return (unsigned)(groups * ((g.ix + LINE_X - 1) / LINE_X));
+}
 
 // Longest segment of the y (dir 1) or z (dir 2) sweep whose state offsets
 // from a thread's column pointer (the cell before the segment) stay below
@@ -993,8 +996,58 @@ inline int lseg_limit(const Geom& g, int dir) {
 }
 inline int clamp_lseg(const Geom& g, int dir, int lseg) { return std::min(lseg, lseg_limit(g, dir)); }
 
+// One line sweep to be cut into segments: workgroups per segment layer and
+// cells along the sweep.
+struct LineWork {
+  int tiles, cells;
+};
+inline LineWork line_work(const Geom& g, int dir) {
+  return {(int)line_tiles(g, dir), dir == 1 ? g.iy : g.iz};
+}
+// Segment length of `cells` cells cut into the fewest segments of at most
+// `lseg`, made equally long.
+inline int even_lseg(int cells, int lseg) {
+  const int n = (cells + lseg - 1) / lseg;
+  return (cells + n - 1) / n;
+}
+// Longest segment of a launch over n line sweeps on `cus` compute units that
+// hold `occ` workgroups each: the length L whose modelled time is least.  A
+// segment costs L cells and about 5 more (the window's first cells, one extra
+// face).  With k workgroups per compute unit the launch lasts
+//   (L + 5) * (max(ceil(k / occ), 0.8 k) + 0.5)
+// cell times of a lone workgroup: k / occ rounds while latency bounds a wave,
+// 0.8 of a cell time per workgroup once the vector units or the memory do, and
+// half a segment of uneven finish.  Short segments fill the chip on small
+// grids, longer ones save the restarts on large ones.  Measured over grids of
+// 32^3 to 256^3, KEEP4 and SLAU6, Euler and NS, both precisions: on average
+// 3%, at most 19%, above the best length found by trying all; always 64 cells
+// took 100 us for a KEEP4 NS y sweep at 64^3 (16 workgroups), this rule's 4
+// cells 16 us; at 256^3 both lie within 2%.
+inline int pick_lseg(const LineWork* p, int n, int occ, int cus) {
+  int longest = 1;
+  for (int m = 0; m < n; ++m) longest = std::max(longest, p[m].cells);
+  int best = longest;
+  double cost = 0.0;
+  for (int parts = 1, last = 0; parts <= longest; ++parts) {
+    const int L = (longest + parts - 1) / parts;
+    if (L == last) continue;
+    last = L;
+    long long blocks = 0;
+    int len = 1;
+    for (int m = 0; m < n; ++m) {
+      const int l = even_lseg(p[m].cells, L);
+      blocks += (long long)p[m].tiles * ((p[m].cells + l - 1) / l);
+      len = std::max(len, l);
+    }
+    const long long k = (blocks + cus - 1) / cus;
+    const double t = (len + 5) * (std::max((double)((k + occ - 1) / occ), 0.8 * (double)k) + 0.5);
+    if (parts == 1 || t < cost) cost = t, best = L;
+  }
+  return best;
+}
+
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO, int DIR, int EP>
-__device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx, int by, int bz) {
+__device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx, int bz) {
   const Prim<S>& P = a.P;
   const Prim<S>& Pn = a.Pn;
   const Geom& g = a.g;
@@ -1004,8 +1057,11 @@ __device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx
   const double cd = a.cd;
   using St = Sten<ORDER, VISC, VO>;
   using CD = CellData<R, DIR, ORDER, SCHEME, VISC, VO>;
-  const int i = g.h + bx * LINE_X + threadIdx.x;
-  const int t = g.h + by * LINE_Y + threadIdx.y;  // k for DIR 1, j for DIR 2
+  const int nbx = (g.ix + LINE_X - 1) / LINE_X;
+  const int pos = bx * LINE_X + threadIdx.x;
+  const int group = DIR == 1 ? pos / g.ix : bx / nbx;
+  const int i = g.h + pos - group * (DIR == 1 ? g.ix : nbx * LINE_X);
+  const int t = g.h + group * LINE_Y + threadIdx.y;  // k for DIR 1, j for DIR 2
   const int s0 = g.h + bz * a.lseg;
   const int nt = DIR == 1 ? g.iz : g.iy;
   const int nd = DIR == 1 ? g.iy : g.iz;
@@ -1145,9 +1201,9 @@ __device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx
 
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO, int DIR, int EP>
 __global__ __launch_bounds__(256) void k_sweep_line(SweepArgs<R, S> a) {
-  int bx, by, bz;
-  launch_tile(bx, by, bz);
-  sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(a, bx, by, bz);
+  const int gx = line_tiles(a.g, DIR);
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(a, t % gx, t / gx);
 }
 
 // Persistent batched y / z sweep over the tiles of several cases.
@@ -1156,9 +1212,8 @@ __global__ __launch_bounds__(256) void k_sweep_line_batch(const SweepArgs<R, S>*
                                                           const TileMap* __restrict__ map, int ncase, int ntiles) {
   for (int t = xcd_tile(blockIdx.x, gridDim.x); t < ntiles; t += gridDim.x) {
     const int ci = find_case(map, ncase, t);
-    const int local = t - map[ci].start, nbx = map[ci].nbx, nby = map[ci].nby;
-    sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(cases[ci], local % nbx, (local / nbx) % nby,
-                                                            local / (nbx * nby));
+    const int local = t - map[ci].start, nbx = map[ci].nbx;
+    sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(cases[ci], local % nbx, local / nbx);
   }
 }
 

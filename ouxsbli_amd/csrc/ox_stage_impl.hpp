@@ -31,12 +31,10 @@ template <int ORDER, int VISC, int VO> dim3 grid_x(const Geom& g) {
 inline dim3 grid_xrow(const Geom& g) {
   return dim3((unsigned)(cdiv(g.iy, XROW_BAND) * g.iz * (XROW_BAND / (256 / g.ix))));
 }
-inline dim3 grid_y(const Geom& g, int lseg) {
-  return dim3(cdiv(g.ix, LINE_X), cdiv(g.iz, LINE_Y), cdiv(g.iy, lseg));
-}
-inline dim3 grid_z(const Geom& g, int lseg) {
-  return dim3(cdiv(g.ix, LINE_X), cdiv(g.iy, LINE_Y), cdiv(g.iz, lseg));
-}
+// k_sweep_line: the tiles of one segment layer after another, in one dimension
+// (a launch's second and third dimensions end at 65535)
+inline dim3 grid_y(const Geom& g, int lseg) { return dim3(line_tiles(g, 1) * cdiv(g.iy, lseg)); }
+inline dim3 grid_z(const Geom& g, int lseg) { return dim3(line_tiles(g, 2) * cdiv(g.iz, lseg)); }
 inline dim3 line_block() { return dim3(LINE_X, LINE_Y, 1); }
 
 // What precedes the sweeps of a stage on one case: primitives when they do not
@@ -168,6 +166,22 @@ void bc_after_erased(const Geom& g, void* const* pn, hipStream_t st) {
   launch_bc_sensors<R, S, ORDER, SCHEME>(g, P, st);
 }
 
+// Workgroups of k_sweep_line one compute unit holds, asked once per kernel.
+template <class R, class S, int ORDER, int SCHEME, int VISC, int VO, int DIR, int EP> int line_occ_of() {
+  static const int occ = [] {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_sweep_line_batch<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>, 256,
+                                                     0) != hipSuccess)
+      n = 1;
+    return std::max(n, 1);
+  }();
+  return occ;
+}
+template <class R, class S, int ORDER, int SCHEME, int VISC, int VO> int line_occ(int dir) {
+  return dir == 1 ? line_occ_of<R, S, ORDER, SCHEME, VISC, VO, 1, EP_RHS>()
+                  : line_occ_of<R, S, ORDER, SCHEME, VISC, VO, 2, EP_RK3_S23>();
+}
+
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO> BatchOps batch_ops() {
   BatchOps o;
   o.args_bytes = sizeof(SweepArgs<R, S>);
@@ -175,6 +189,7 @@ template <class R, class S, int ORDER, int SCHEME, int VISC, int VO> BatchOps ba
   o.prepare = &prepare_stage<R, S, ORDER, SCHEME, VISC, VO>;
   o.make_args = &make_sweep_args_erased<R, S>;
   o.launch = &run_stage_batch<R, S, ORDER, SCHEME, VISC, VO>;
+  o.line_occ = &line_occ<R, S, ORDER, SCHEME, VISC, VO>;
   o.bc_after = &bc_after_erased<R, S, ORDER, SCHEME, VISC>;
   return o;
 }
