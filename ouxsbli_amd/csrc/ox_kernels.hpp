@@ -305,20 +305,24 @@ __device__ __forceinline__ void cross_fields(const Prim<S>& P, const Geom& g, co
   }
 }
 
-// Issues the loads of cell m (sensor read at ms, its periodic image).
+// Issues the loads of cell m (sensor read at ms, its periodic image): its own
+// values, and the transverse stencil values of a viscous run.
 template <class S, int DIR, int ORDER, int SCHEME, int VISC, int VO, bool LOAD_S = true>
-__device__ __forceinline__ void fetch_cell(const Prim<S>& P, const Geom& g, int m, int ms, RawCell<S, VISC, VO>& r) {
+__device__ __forceinline__ void fetch_values(const Prim<S>& P, int m, int ms, RawCell<S, VISC, VO>& r) {
   r.rho = G(P.rho)[m];
   r.u = G(P.u)[m];
   r.v = G(P.v)[m];
   r.w = G(P.w)[m];
   r.p = G(P.p)[m];
   if constexpr (LOAD_S && kUsesSensor<SCHEME, ORDER>) r.s = G(P.s)[ms];
+  if constexpr (VISC == 2) {
+    r.mt = G(P.mut)[m];
+    r.qc2 = G(P.qc2)[m];
+  }
+}
+template <class S, int DIR, int VISC, int VO>
+__device__ __forceinline__ void fetch_cross(const Prim<S>& P, const Geom& g, int m, RawCell<S, VISC, VO>& r) {
   if constexpr (VISC) {
-    if constexpr (VISC == 2) {
-      r.mt = G(P.mut)[m];
-      r.qc2 = G(P.qc2)[m];
-    }
     const S* f[4];
     int st[4];
     cross_fields<S, DIR>(P, g, f, st);
@@ -332,6 +336,11 @@ __device__ __forceinline__ void fetch_cell(const Prim<S>& P, const Geom& g, int 
       }
     }
   }
+}
+template <class S, int DIR, int ORDER, int SCHEME, int VISC, int VO, bool LOAD_S = true>
+__device__ __forceinline__ void fetch_cell(const Prim<S>& P, const Geom& g, int m, int ms, RawCell<S, VISC, VO>& r) {
+  fetch_values<S, DIR, ORDER, SCHEME, VISC, VO, LOAD_S>(P, m, ms, r);
+  fetch_cross<S, DIR, VISC, VO>(P, g, m, r);
 }
 
 // cross_d over the raw stencil values (centre entry zero, never read)
@@ -1046,8 +1055,44 @@ inline int pick_lseg(const LineWork* p, int n, int occ, int cus) {
   return best;
 }
 
+// The viscous part of a line sweep's window in LDS, a ring of SW cells per
+// thread (FP64 NS): the cross derivatives, mu and (unless the convective flux
+// reads it) T.  Only the viscous half of a face reads these values, so they need
+// not sit in registers through the convective half nor be moved from face to
+// face.  That and loading a face's operands after its convective half (below)
+// let the SLAU6 NS sweeps run two waves per SIMD (254 and 256 registers; with
+// the whole window in registers 368 and 416, one wave) on 74 KB of LDS per
+// workgroup, with 13% fewer vector instructions.  The sweeps are bound by the
+// vector units (y, 0.73 busy) and by memory (z).  Best segment length on either
+// side: at 256^3 y 764 -> 700, z 1091 -> 1036 us; at 192^3 y 425 -> 355, z 538 ->
+// 461 us; KEEP4 NS at 64^3 y 18 -> 16, z 23 -> 21 us.  FP32 windows fit two to
+// four waves as they are, and their ring was slower (SLAU6 NS at 128^3: y 58 ->
+// 62, z 87 -> 88 us).  LES stays in registers at one wave: with its ring (mt and H
+// as well) the FP64 z sweep spilled and took 780 us where it takes 691 (Hybrid6
+// at 192^3).
+template <class R, int SCHEME, int VISC> constexpr int ring_fields() {
+  return VISC != 1 || sizeof(R) != 8 ? 0 : kUsesT<SCHEME> ? 5 : 6;  // d1..d4, mu[, T]
+}
+template <class R, int ORDER, int SCHEME, int VISC, int VO> constexpr int ring_values() {
+  return ring_fields<R, SCHEME, VISC>() * Sten<ORDER, VISC, VO>::SW * 256;
+}
+template <int ORDER, int SCHEME, int VISC, int VO, class R, class CD>
+__device__ __forceinline__ void ring_put(R* p, const CD& d) {
+  constexpr int st = Sten<ORDER, VISC, VO>::SW * 256;  // one field
+  p[0] = d.d1; p[st] = d.d2; p[2 * st] = d.d3; p[3 * st] = d.d4; p[4 * st] = d.mu;
+  if constexpr (!kUsesT<SCHEME>) p[5 * st] = d.T;
+}
+template <int ORDER, int SCHEME, int VISC, int VO, class R, class CD>
+__device__ __forceinline__ void ring_get(const R* p, CD& d) {
+  constexpr int st = Sten<ORDER, VISC, VO>::SW * 256;
+  d.d1 = p[0]; d.d2 = p[st]; d.d3 = p[2 * st]; d.d4 = p[3 * st]; d.mu = p[4 * st];
+  if constexpr (!kUsesT<SCHEME>) d.T = p[5 * st];
+}
+// waves per SIMD a line sweep's registers are held to
+template <int VISC> constexpr int line_waves() { return VISC == 2 ? 1 : 2; }
+
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO, int DIR, int EP>
-__device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx, int bz) {
+__device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx, int bz, R* ring) {
   const Prim<S>& P = a.P;
   const Prim<S>& Pn = a.Pn;
   const Geom& g = a.g;
@@ -1098,12 +1143,16 @@ __device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx
     return sp < g.h ? sp + period : (sp >= g.h + nd ? sp - period : sp);
   };
   using RC = RawCell<S, VISC, VO>;
+  constexpr bool RING = ring_fields<R, SCHEME, VISC>() > 0;
+  R* mine = ring + threadIdx.x + LINE_X * threadIdx.y;
   CD win[St::SW];
 #pragma unroll
   for (int m = 0; m < St::SW - 1; ++m) {
     const int sp = s0 - St::HW + m;
     load_cell<R, S, DIR, ORDER, SCHEME, VISC, VO>(P, g, c, mbase + sp * stride, mbase + wrap(sp) * stride, win[m]);
+    if constexpr (RING) ring_put<ORDER, SCHEME, VISC, VO>(mine + m * 256, win[m]);
   }
+  int head = 0;  // ring slot of the window's first cell
   // Software pipeline: the values of the cell that enters the window at face
   // f+1, and the residual (and state) of the cell that face f+1 completes,
   // are loaded while face f is computed, so that one face's arithmetic
@@ -1115,27 +1164,52 @@ __device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx
   }
   R Fp[5];
   CellState<DIR, EP> cs;
-  // The prefetches below are issued on every iteration, the last one included
-  // (its values are never used): a prefetch behind a branch makes the
-  // compiler wait for every outstanding memory operation, the residual stores
-  // of the iteration included, at the loop's merge points.  On the last
-  // iteration the cell entering the window is clamped to the array's last
-  // layer along DIR, and cell f+1 = s_end is at most that layer as well.
+  // Software pipeline.  The values of the cell that enters the window at face
+  // f+1 are loaded while face f is computed.  Windows held in registers through
+  // a viscous face issue its transverse stencils, and the state of the cell that
+  // face f+1 completes, a whole face ahead.  With the ring the state of cell f,
+  // which face f completes, and the next cell's stencils are issued between the
+  // two halves of face f, so that those registers are free during the convective
+  // half; Euler sweeps load the state of cell f at the top of the iteration.
+  // The loads are issued on every iteration, the last one included (its
+  // values are never used): a load behind a branch makes the compiler wait
+  // for every outstanding memory operation, the residual stores of the
+  // iteration included, at the loop's merge points.  On the last iteration
+  // the cell entering the window is clamped to the array's last layer along
+  // DIR, and cell f+1 = s_end is at most that layer as well; on the first, cell
+  // f = s0 - 1 is at least layer 0.
+  constexpr bool AHEAD = VISC && !RING;
   const int n_along = DIR == 1 ? g.ny : g.nz;
   for (int f = s0 - 1; f < s_end; ++f) {
     finish_cell<R, S, DIR, ORDER, SCHEME, VISC, VO>(g, c, nxt, win[St::SW - 1]);
-    {
-      const int sp = min(f + 1 + St::HW, n_along - 1);
-      fetch_cell<S, DIR, ORDER, SCHEME, VISC, VO>(P, g, mbase + sp * stride, mbase + wrap(sp) * stride, nxt);
-    }
-    // residual (and state) of cell f+1, consumed one iteration later
-    CellState<DIR, EP> ncs;
+    if constexpr (RING)
+      ring_put<ORDER, SCHEME, VISC, VO>(mine + (head == 0 ? St::SW - 1 : head - 1) * 256, win[St::SW - 1]);
+    const int sp = min(f + 1 + St::HW, n_along - 1);
+    fetch_values<S, DIR, ORDER, SCHEME, VISC, VO>(P, mbase + sp * stride, mbase + wrap(sp) * stride, nxt);
+    if constexpr (AHEAD) fetch_cross<S, DIR, VISC, VO>(P, g, mbase + sp * stride, nxt);
     const int q = (f - s0 + 1) * qstride;  // cell f, from the column pointers
-    fetch_state<DIR, EP>(Racc, sa, q + qstride, g.nx, ncs);
-    const double *Ra = cs.R, *Qa = cs.A, *Qb = cs.B, *Qc = cs.C;
+    CellState<DIR, EP> ncs;
+    if constexpr (AHEAD) fetch_state<DIR, EP>(Racc, sa, q + qstride, g.nx, ncs);
+    if constexpr (!VISC) fetch_state<DIR, EP>(Racc, sa, q, g.nx, cs);
     R F[5];
-    face_flux<R, DIR, ORDER, SCHEME, VISC, VO>(c, tvd, variant, inv_d, win, F);
+    face_conv<R, DIR, ORDER, SCHEME, VISC, VO>(c, tvd, variant, win, F);
+    if constexpr (RING) {
+      OX_SPLIT_FENCE();
+      fetch_state<DIR, EP>(Racc, sa, q, g.nx, cs);
+      fetch_cross<S, DIR, VISC, VO>(P, g, mbase + sp * stride, nxt);
+      CD vw[St::SW];
+#pragma unroll
+      for (int m = 0; m < St::SW; ++m) {
+        vw[m] = win[m];
+        ring_get<ORDER, SCHEME, VISC, VO>(mine + (head + m >= St::SW ? head + m - St::SW : head + m) * 256, vw[m]);
+      }
+      face_visc<R, DIR, ORDER, SCHEME, VISC, VO>(c, inv_d, vw, F);
+      head = head + 1 == St::SW ? 0 : head + 1;
+    } else {
+      face_visc<R, DIR, ORDER, SCHEME, VISC, VO>(c, inv_d, win, F);
+    }
     if (f >= s0) {
+      const double *Ra = cs.R, *Qa = cs.A, *Qb = cs.B, *Qc = cs.C;
       double Rl[5];
 #pragma unroll
       for (int l = 0; l < 5; ++l) Rl[l] = Ra[l] + cd * (-(double)Fp[l] + (double)F[l]);
@@ -1195,25 +1269,27 @@ __device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx
     for (int l = 0; l < 5; ++l) Fp[l] = F[l];
 #pragma unroll
     for (int m = 0; m < St::SW - 1; ++m) win[m] = win[m + 1];
-    cs = ncs;
+    if constexpr (AHEAD) cs = ncs;
   }
 }
 
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO, int DIR, int EP>
-__global__ __launch_bounds__(256) void k_sweep_line(SweepArgs<R, S> a) {
+__global__ __launch_bounds__(256, line_waves<VISC>()) void k_sweep_line(SweepArgs<R, S> a) {
+  __shared__ R ring[std::max(1, ring_values<R, ORDER, SCHEME, VISC, VO>())];
   const int gx = line_tiles(a.g, DIR);
   const int t = xcd_tile(blockIdx.x, gridDim.x);
-  sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(a, t % gx, t / gx);
+  sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(a, t % gx, t / gx, ring);
 }
 
 // Persistent batched y / z sweep over the tiles of several cases.
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO, int DIR, int EP>
-__global__ __launch_bounds__(256) void k_sweep_line_batch(const SweepArgs<R, S>* __restrict__ cases,
-                                                          const TileMap* __restrict__ map, int ncase, int ntiles) {
+__global__ __launch_bounds__(256, line_waves<VISC>()) void k_sweep_line_batch(
+    const SweepArgs<R, S>* __restrict__ cases, const TileMap* __restrict__ map, int ncase, int ntiles) {
+  __shared__ R ring[std::max(1, ring_values<R, ORDER, SCHEME, VISC, VO>())];
   for (int t = xcd_tile(blockIdx.x, gridDim.x); t < ntiles; t += gridDim.x) {
     const int ci = find_case(map, ncase, t);
     const int local = t - map[ci].start, nbx = map[ci].nbx;
-    sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(cases[ci], local % nbx, local / nbx);
+    sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(cases[ci], local % nbx, local / nbx, ring);
   }
 }
 
