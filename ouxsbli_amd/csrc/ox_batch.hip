@@ -71,7 +71,7 @@ struct BCase {
 };
 
 // Cases sharing a kernel specialisation.  3-D groups launch three sweeps per
-// stage (LES groups first the SGS viscosity and its two ghost-copy passes);
+// stage (LES groups first the SGS viscosity);
 // 2-D groups one fused stage kernel (launch2[stage]).
 struct BGroup {
   int dim, prec, key, rk;
@@ -214,16 +214,16 @@ int build_plan(ox_batch* b) {
     }
   }
   // tile maps: per 3-D group, per direction, one TileMap per member (LES
-  // groups: three more, for the SGS viscosity and the two ghost-copy
-  // passes); 2-D groups count their tiles (the case lookup reads the
-  // descriptors)
+  // groups: one more, for the SGS viscosity); 2-D groups count their tiles
+  // (the case lookup reads the descriptors)
   std::vector<ox::TileMap> maps;
-  std::vector<size_t> map_off;  // per group: index of its x map (y at +n, z at +2n, LES at +3n..+5n)
-  std::vector<std::array<int, 3>> ntiles, ntiles_les;
+  std::vector<size_t> map_off;  // per group: index of its x map (y at +n, z at +2n, LES at +3n)
+  std::vector<std::array<int, 3>> ntiles;
+  std::vector<int> ntiles_les;
   for (BGroup& G : b->groups) {
     map_off.push_back(maps.size());
     std::array<int, 3> nt{0, 0, 0};
-    std::array<int, 3> nl{0, 0, 0};
+    int nl = 0;
     if (G.dim == 2) {
       for (BCase* c : G.members) nt[0] += c->s2->ntiles;
       ntiles.push_back(nt);
@@ -253,23 +253,12 @@ int build_plan(ox_batch* b) {
     }
     ntiles.push_back(nt);
     if (G.les) {
-      for (int d = 0; d < 3; ++d) {
-        for (BCase* c : G.members) {
-          const ox::Geom& g = c->s->C.g;
-          ox::TileMap m{};
-          if (d == 0) {  // 64 x 4 cells of one plane, as k_les_mut's blocks
-            m.nbx = (int)cdivu(g.nx - 2, 64);
-            m.nby = (int)cdivu(g.ny - 2, 4);
-            m.nbz = g.nz - 2;
-          } else {  // 256 items of a ghost-copy pass
-            m.nbx = (int)cdivu(ox::les_bc_items(g, d - 1), 256);
-            m.nby = 1;
-            m.nbz = 1;
-          }
-          m.start = nl[d];
-          nl[d] += m.nbx * m.nby * m.nbz;
-          maps.push_back(m);
-        }
+      for (BCase* c : G.members) {
+        ox::TileMap m{};
+        ox::les_tiles(c->s->C.g, m.nbx, m.nby, m.nbz);
+        m.start = nl;
+        nl += m.nbx * m.nby * m.nbz;
+        maps.push_back(m);
       }
     }
     ntiles_les.push_back(nl);
@@ -299,11 +288,11 @@ int build_plan(ox_batch* b) {
           L.map[d] = b->d_map + map_off[gi] + (size_t)d * n;
           L.ntiles[d] = ntiles[gi][d];
           L.grid[d] = std::max(1, std::min(ntiles[gi][d], kMaxGrid));
-          if (G.les) {
-            L.map_les[d] = b->d_map + map_off[gi] + (size_t)(3 + d) * n;
-            L.ntiles_les[d] = ntiles_les[gi][d];
-            L.grid_les[d] = std::max(1, std::min(ntiles_les[gi][d], kMaxGrid));
-          }
+        }
+        if (G.les) {
+          L.map_les = b->d_map + map_off[gi] + (size_t)3 * n;
+          L.ntiles_les = ntiles_les[gi];
+          L.grid_les = std::max(1, std::min(ntiles_les[gi], kMaxGrid));
         }
       } else {
         L.ntiles[0] = ntiles[gi][0];

@@ -69,6 +69,23 @@ template <int ORDER, int VISC, int VO> struct Sten {
   static constexpr int VH = vcross<VO>() / 2;  // half width of the cross-derivative stencil
 };
 
+// Workgroups are dispatched round-robin over the eight XCDs, and each XCD has
+// its own L2.  For n workgroups with n a multiple of 8, tile
+// (b % 8) * (n / 8) + b / 8 gives XCD b % 8 one contiguous run of n / 8
+// tiles, so the tiles whose stencils overlap (neighbours along the second and
+// third launch dimensions) share an L2 instead of fetching the same rows into
+// two.  The map is a permutation of [0, n).
+#ifndef OX_XCD_SWIZZLE
+#define OX_XCD_SWIZZLE 1
+#endif
+#ifndef OX_XSWEEP_ZMAJOR
+#define OX_XSWEEP_ZMAJOR 1
+#endif
+__device__ __forceinline__ int xcd_tile(int b, int n) {
+  if (!OX_XCD_SWIZZLE || (n & 7)) return b;
+  return (b & 7) * (n >> 3) + (b >> 3);
+}
+
 // state index of (i,l,j,k), 0-based: 64-bit, since the state holds five
 // values per cell and a grid of up to 2^31 cells fits one GPU's HBM (the
 // bracket, 5 * (j + ny * k) + l, stays below 5 * ny * nz)
@@ -125,15 +142,40 @@ __global__ __launch_bounds__(256) void k_prim(const double* __restrict__ QJ, Pri
 
 // ---------------------------------------------------------------------------
 // Selective mixed-scale SGS viscosity (calc_mut, 3D_solver/src/calc_les.f90:
-// 12-125) over the cells the reference computes (Fortran 2..n-1).  Only the
-// seven test-filtered values the central differences and qc2 read are formed
-// (the centre and its six face neighbours); exponents 1/4 as sqrt(sqrt(.)).
+// 12-125) over the cells the reference computes (Fortran 2..n-1), exponents 1/4
+// as sqrt(sqrt(.)), and its ghost cells (set_bc_mut_common,
+// 3D_solver/src/set_bc_common.f90:296-335).
+//
+// A cell reads the test-filtered velocity at itself and its six face neighbours,
+// each a seven-point stencil.  A workgroup takes LES_X x LES_Y columns and walks
+// les_seg planes: every plane is filtered once, tile and rim, into LDS, and the
+// cells of the plane before read the three planes around theirs (four slots, so
+// one barrier per plane).  Each thread keeps its column's last planes, and their
+// in-plane neighbours, in registers.  That is 1.3 filter evaluations per cell and
+// velocity component instead of seven, and 24 loads per cell instead of 168.
+// Bound by latency and the vector units.  Each cell filtering its seven points by
+// itself, and two launches for the ghost cells, took at 192^3 484 us in FP64 and
+// 232 us in FP32; this takes 237 and 148 us (96^3: 70 -> 45 and 37 -> 26 us).
 // ---------------------------------------------------------------------------
-template <class S, class R>
-__device__ __forceinline__ R tfilt(const S* __restrict__ f, int m, int sy, int sz) {
-  const R c0 = R(G(f)[m]);
-  return c0 + R(0.25) * (R(G(f)[m - 1]) - R(2) * c0 + R(G(f)[m + 1]) + R(G(f)[m - sy]) - R(2) * c0 +
-                         R(G(f)[m + sy]) + R(G(f)[m - sz]) - R(2) * c0 + R(G(f)[m + sz]));
+constexpr int LES_X = 32, LES_Y = 8;
+// Planes per workgroup: eight, or four where eight leave less than two
+// workgroups per CU (at 64^3, FP64: eight 28 us, four 23 us; at 192^3 246 and 270).
+__host__ __device__ inline int les_seg(const Geom& g) {
+  const long long n = (long long)((g.nx - 2 + LES_X - 1) / LES_X) * ((g.ny - 2 + LES_Y - 1) / LES_Y) * ((g.nz - 2 + 7) / 8);
+  return n < 512 ? 4 : 8;
+}
+// workgroups along x, y, z over the computed cells
+inline void les_tiles(const Geom& g, int& bx, int& by, int& bz) {
+  bx = (g.nx - 2 + LES_X - 1) / LES_X;
+  by = (g.ny - 2 + LES_Y - 1) / LES_Y;
+  bz = (g.nz - 2 + les_seg(g) - 1) / les_seg(g);
+}
+
+// The test filter at one point from its centre and its neighbours in the order
+// -x, +x, -y, +y, -z, +z.
+template <class R>
+__device__ __forceinline__ R tfilt(R c0, R xm, R xp, R ym, R yp, R zm, R zp) {
+  return c0 + R(0.25) * (xm - R(2) * c0 + xp + ym - R(2) * c0 + yp + zm - R(2) * c0 + zp);
 }
 
 template <class R>
@@ -150,28 +192,30 @@ __device__ __forceinline__ void grad9(R um, R up, R vm, R vp, R wm, R wp, R dx, 
   g[8] = R(0.5) * (-wz[0] + wz[1]) * dz;
 }
 
-// nu_t and qc2 of cell (i, j, k), 1 <= i <= nx-2, 1 <= j <= ny-2, 1 <= k <= nz-2.
+// The filtered velocity of LES_Y x LES_X columns and a rim of one, four planes.
+template <class R> using LesPlanes = R[4][3][LES_Y + 2][LES_X + 2];
+
+// nu_t and qc2 of cell (i, j, k), 1 <= i <= nx-2, 1 <= j <= ny-2, 1 <= k <= nz-2,
+// and of the ghost cells that copy it, from the velocities at the cell and its
+// neighbours (centre, -x, +x, -y, +y, -z, +z) and the filtered planes (the cell at
+// (px, py), plane k in slot k % 4).
 template <class S, class R>
 __device__ __forceinline__ void les_mut_cell(const Prim<S>& P, const Geom& g, const PhysC<R>& c, int i, int j,
-                                             int k) {
-  const int sy = g.nx, sz = g.nx * g.ny;
+                                             int k, const R (&raw)[3][7], int px, int py,
+                                             const LesPlanes<R>& pl) {
   const int m = cidx(g, i, j, k);
+  // cells next to the outermost layer are not filtered
   const bool filt = (i >= 2 && i <= g.nx - 3 && j >= 2 && j <= g.ny - 3 && k >= 2 && k <= g.nz - 3);
-  const S* U[3] = {P.u, P.v, P.w};
-  R raw[3][7], fil[3][7];  // centre, -x, +x, -y, +y, -z, +z
-  const int off[7] = {0, -1, 1, -sy, sy, -sz, sz};
-  // The filter is formed at every stencil point whatever `filt` says, around
-  // the centre itself where the cell is not filtered (its neighbours always
-  // exist there; the value is not used), so that all loads sit in one block
-  // the compiler can issue ahead of their use instead of one branch per point.
+  R fil[3][7];
 #pragma unroll
-  for (int f = 0; f < 3; ++f)
+  for (int f = 0; f < 3; ++f) {
+    const auto& pm = pl[(k - 1) & 3][f];
+    const auto& pc = pl[k & 3][f];
+    const auto& pp = pl[(k + 1) & 3][f];
+    const R ft[7] = {pc[py][px], pc[py][px - 1], pc[py][px + 1], pc[py - 1][px], pc[py + 1][px], pm[py][px], pp[py][px]};
 #pragma unroll
-    for (int t = 0; t < 7; ++t) {
-      raw[f][t] = R(G(U[f])[m + off[t]]);
-      const R ft = tfilt<S, R>(U[f], filt ? m + off[t] : m, sy, sz);
-      fil[f][t] = filt ? ft : raw[f][t];
-    }
+    for (int t = 0; t < 7; ++t) fil[f][t] = filt ? ft[t] : raw[f][t];
+  }
   const R dx = R(g.inv_dx), dy = R(g.inv_dy), dz = R(g.inv_dz);
   R gr[9], gh[9];
   {
@@ -205,72 +249,115 @@ __device__ __forceinline__ void les_mut_cell(const Prim<S>& P, const Geom& g, co
                ((gr[3] + gr[1]) * (gr[3] + gr[1]) + (gr[7] + gr[5]) * (gr[7] + gr[5]) +
                 (gr[2] + gr[6]) * (gr[2] + gr[6]));
   const R nut = ftheta * R(0.06) * fsqrt(fsqrt(S2)) * fsqrt(fsqrt(q2)) * c.les_delta15;
-  G(P.qc2)[m] = (S)q2;
-  G(P.mut)[m] = (S)(R(G(P.rho)[m]) * nut);
-}
-
-template <class S, class R>
-__global__ __launch_bounds__(256) void k_les_mut(Prim<S> P, Geom g, PhysC<R> c) {
-  const int i = 1 + blockIdx.x * 64 + threadIdx.x;
-  const int j = 1 + blockIdx.y * 4 + threadIdx.y;
-  const int k = 1 + blockIdx.z;
-  if (i > g.nx - 2 || j > g.ny - 2) return;
-  les_mut_cell<S, R>(P, g, c, i, j, k);
-}
-
-// set_bc_mut_common (3D_solver/src/set_bc_common.f90:296-335): pass 0 = x
-// faces, y faces and xy corners over k = Fortran 2..nz-1; pass 1 = z planes.
-// Item t of a pass (items past the pass's count do nothing); pass 1 reads
-// what pass 0 wrote, so the two run as separate launches.
-template <class S>
-__device__ __forceinline__ void les_bc_item(const Prim<S>& P, const Geom& g, int pass, long long t) {
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  __attribute__((address_space(1))) S* A[2] = {G(P.mut), G(P.qc2)};
-  if (pass == 0) {
-    const int nk = nz - 2;
-    const long long nxf = (long long)(ny - 2) * nk, nyf = (long long)(nx - 2) * nk;
-    if (t < nxf) {
-      const int j = 1 + (int)(t % (ny - 2)), k = 1 + (int)(t / (ny - 2));
-      for (int a = 0; a < 2; ++a) {
-        A[a][cidx(g, 0, j, k)] = A[a][cidx(g, nx - 2, j, k)];
-        A[a][cidx(g, nx - 1, j, k)] = A[a][cidx(g, 1, j, k)];
-      }
-    } else if (t < nxf + nyf) {
-      const long long u = t - nxf;
-      const int i = 1 + (int)(u % (nx - 2)), k = 1 + (int)(u / (nx - 2));
-      for (int a = 0; a < 2; ++a) {
-        A[a][cidx(g, i, 0, k)] = A[a][cidx(g, i, ny - 2, k)];
-        A[a][cidx(g, i, ny - 1, k)] = A[a][cidx(g, i, 1, k)];
-      }
-    } else if (t < nxf + nyf + nk) {
-      const int k = 1 + (int)(t - nxf - nyf);
-      for (int a = 0; a < 2; ++a) {
-        A[a][cidx(g, 0, 0, k)] = A[a][cidx(g, nx - 2, ny - 2, k)];
-        A[a][cidx(g, nx - 1, 0, k)] = A[a][cidx(g, 1, ny - 2, k)];
-        A[a][cidx(g, 0, ny - 1, k)] = A[a][cidx(g, nx - 2, 1, k)];
-        A[a][cidx(g, nx - 1, ny - 1, k)] = A[a][cidx(g, 1, 1, k)];
-      }
-    }
-  } else {
-    if (t < (long long)nx * ny) {
-      const int i = (int)(t % nx), j = (int)(t / nx);
-      for (int a = 0; a < 2; ++a) {
-        A[a][cidx(g, i, j, 0)] = A[a][cidx(g, i, j, nz - 2)];
-        A[a][cidx(g, i, j, nz - 1)] = A[a][cidx(g, i, j, 1)];
+  const S qv = (S)q2, mv = (S)(R(G(P.rho)[m]) * nut);
+  G(P.qc2)[m] = qv;
+  G(P.mut)[m] = mv;
+  // the outermost layer along each direction copies the cell one layer inside
+  // the opposite end: up to seven copies of this cell
+  const int ai = i == 1 ? g.nx - 1 : (i == g.nx - 2 ? 0 : -1);
+  const int aj = j == 1 ? g.ny - 1 : (j == g.ny - 2 ? 0 : -1);
+  const int ak = k == 1 ? g.nz - 1 : (k == g.nz - 2 ? 0 : -1);
+  if (ai >= 0 || aj >= 0 || ak >= 0) {
+    const int xs[2] = {i, ai}, ys[2] = {j, aj}, zs[2] = {k, ak};
+    for (int c3 = 1; c3 < 8; ++c3) {
+      const int x = xs[c3 & 1], y = ys[(c3 >> 1) & 1], z = zs[(c3 >> 2) & 1];
+      if (x >= 0 && y >= 0 && z >= 0) {
+        G(P.qc2)[cidx(g, x, y, z)] = qv;
+        G(P.mut)[cidx(g, x, y, z)] = mv;
       }
     }
   }
 }
 
-template <class S>
-__global__ __launch_bounds__(256) void k_les_bc(Prim<S> P, Geom g, int pass) {
-  les_bc_item<S>(P, g, pass, (long long)blockIdx.x * 256 + threadIdx.x);
+// One workgroup's columns and planes (blocks of 256 threads).
+template <class S, class R>
+__device__ __forceinline__ void les_mut_tile(const Prim<S>& P, const Geom& g, const PhysC<R>& c, int bx, int by, int bz,
+                                             LesPlanes<R>& pl) {
+  const int sy = g.nx, sz = g.nx * g.ny;
+  const int i0 = 1 + bx * LES_X, j0 = 1 + by * LES_Y, k0 = 1 + bz * les_seg(g);
+  const int k1 = min(k0 + les_seg(g), g.nz - 1);  // cells of planes k0 .. k1 - 1
+  const int tid = threadIdx.x, tx = tid % LES_X, ty = tid / LES_X;
+  const int i = i0 + tx, j = j0 + ty;
+  const bool inside = i <= g.nx - 2 && j <= g.ny - 2;
+  const S* U[3] = {P.u, P.v, P.w};
+  // the rim's points (its corners are not read): the rows below and above the
+  // tile, then the columns left and right of it, one per thread
+  constexpr int RIM = 2 * LES_X + 2 * LES_Y;
+  static_assert(RIM <= 256, "one rim point per thread");
+  int rx = 0, ry = 0;
+  if (tid < 2 * LES_X) rx = 1 + tid % LES_X, ry = tid < LES_X ? 0 : LES_Y + 1;
+  else rx = tid < 2 * LES_X + LES_Y ? 0 : LES_X + 1, ry = 1 + tid % LES_Y;
+  const int ri = i0 - 1 + rx, rj = j0 - 1 + ry;
+  const bool rim = tid < RIM && ri >= 1 && ri <= g.nx - 2 && rj >= 1 && rj <= g.ny - 2;
+  // this thread's column (a corner's where it has none): the velocities of planes
+  // kk - 2 .. kk + 1 and the in-plane neighbours of planes kk - 1 .. kk + 1, the
+  // last loaded a plane ahead of their use
+  const int col = inside ? cidx(g, i, j, 0) : cidx(g, 1, 1, 0), rcol = rim ? cidx(g, ri, rj, 0) : 0;
+  R z2[3], z1[3], z0[3], zp[3], n1[3][4], n0[3][4], np[3][4];
+  auto neighbours = [&](int m) {
+#pragma unroll
+    for (int f = 0; f < 3; ++f) {
+      np[f][0] = R(G(U[f])[m - 1]);
+      np[f][1] = R(G(U[f])[m + 1]);
+      np[f][2] = R(G(U[f])[m - sy]);
+      np[f][3] = R(G(U[f])[m + sy]);
+    }
+  };
+  neighbours(col + (k0 - 1) * sz);
+#pragma unroll
+  for (int f = 0; f < 3; ++f) {
+    z2[f] = z1[f] = R(0);
+    z0[f] = R(G(U[f])[col + max(k0 - 2, 0) * sz]);
+    zp[f] = R(G(U[f])[col + (k0 - 1) * sz]);
+  }
+  for (int kk = k0 - 1; kk <= k1; ++kk) {
+#pragma unroll
+    for (int f = 0; f < 3; ++f) {
+      z2[f] = z1[f];
+      z1[f] = z0[f];
+      z0[f] = zp[f];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) n1[f][t] = n0[f][t], n0[f][t] = np[f][t];
+    }
+    const int next = col + min(kk + 1, g.nz - 1) * sz;
+#pragma unroll
+    for (int f = 0; f < 3; ++f) zp[f] = R(G(U[f])[next]);
+    neighbours(next);
+    // filtered plane kk where the filter's stencil exists
+    if (kk >= 1 && kk <= g.nz - 2) {
+      if (inside) {
+#pragma unroll
+        for (int f = 0; f < 3; ++f)
+          pl[kk & 3][f][ty + 1][tx + 1] = tfilt<R>(z0[f], n0[f][0], n0[f][1], n0[f][2], n0[f][3], z1[f], zp[f]);
+      }
+      if (rim) {
+        const int m = rcol + kk * sz;
+#pragma unroll
+        for (int f = 0; f < 3; ++f)
+          pl[kk & 3][f][ry][rx] =
+              tfilt<R>(R(G(U[f])[m]), R(G(U[f])[m - 1]), R(G(U[f])[m + 1]), R(G(U[f])[m - sy]), R(G(U[f])[m + sy]),
+                       R(G(U[f])[m - sz]), R(G(U[f])[m + sz]));
+      }
+    }
+    __syncthreads();
+    if (kk > k0 && inside) {
+      R raw[3][7];
+#pragma unroll
+      for (int f = 0; f < 3; ++f) {
+        raw[f][0] = z1[f];
+        raw[f][1] = n1[f][0]; raw[f][2] = n1[f][1]; raw[f][3] = n1[f][2]; raw[f][4] = n1[f][3];
+        raw[f][5] = z2[f]; raw[f][6] = z0[f];
+      }
+      les_mut_cell<S, R>(P, g, c, i, j, kk - 1, raw, tx + 1, ty + 1, pl);
+    }
+  }
 }
 
-// Items of the two passes of les_bc_item over a grid.
-inline long long les_bc_items(const Geom& g, int pass) {
-  return pass == 0 ? (long long)(g.ny - 2) * (g.nz - 2) + (long long)(g.nx - 2) * (g.nz - 2) + (g.nz - 2)
-                   : (long long)g.nx * g.ny;
+template <class S, class R>
+__global__ __launch_bounds__(256) void k_les_mut(Prim<S> P, Geom g, PhysC<R> c, int nbx, int nby) {
+  __shared__ LesPlanes<R> pl;
+  const int t = xcd_tile(blockIdx.x, gridDim.x);
+  les_mut_tile<S, R>(P, g, c, t % nbx, (t / nbx) % nby, t / (nbx * nby), pl);
 }
 
 // ---------------------------------------------------------------------------
@@ -487,23 +574,6 @@ struct TileMap {
   int nbx, nby;  // tiles along the three launch dimensions
   int nbz;
 };
-
-// Workgroups are dispatched round-robin over the eight XCDs, and each XCD has
-// its own L2.  For n workgroups with n a multiple of 8, tile
-// (b % 8) * (n / 8) + b / 8 gives XCD b % 8 one contiguous run of n / 8
-// tiles, so the tiles whose stencils overlap (neighbours along the second and
-// third launch dimensions) share an L2 instead of fetching the same rows into
-// two.  The map is a permutation of [0, n).
-#ifndef OX_XCD_SWIZZLE
-#define OX_XCD_SWIZZLE 1
-#endif
-#ifndef OX_XSWEEP_ZMAJOR
-#define OX_XSWEEP_ZMAJOR 1
-#endif
-__device__ __forceinline__ int xcd_tile(int b, int n) {
-  if (!OX_XCD_SWIZZLE || (n & 7)) return b;
-  return (b & 7) * (n >> 3) + (b >> 3);
-}
 
 // The x sweep's tiles (bx, row band by, plane bz) in x, z, y order under
 // xcd_tile: one XCD's run covers a band of rows through many planes, so both
@@ -773,7 +843,8 @@ __global__ __launch_bounds__(256) void k_sweep_x(SweepArgs<R, S> a) {
 // once a z-sweep epilogue has written the primitive set, so both tiles give
 // the same bits.  Used for such primitive sets only (k_prim takes the ghost
 // layers of an uploaded state as they are), on fully periodic grids, without
-// LES (its ghost SGS fields come from k_les_bc), and not for ORDER 2 with the
+// LES (the ghost SGS fields are copies of the layer next to
+// the boundary), and not for ORDER 2 with the
 // sensor, whose ghost cells copy the adjacent interior sensor
 // (calc_hybrid.f90:54-71) instead of the image's.
 // ---------------------------------------------------------------------------
@@ -1294,32 +1365,18 @@ __global__ __launch_bounds__(256, line_waves<VISC>()) void k_sweep_line_batch(
 }
 
 // Persistent batched SGS viscosity of LES cases over the tiles of several
-// cases (tile = 64 x 4 cells of one plane, the single-case launch's block),
-// reading each case's x-sweep descriptor: the primitive set the stage reads,
-// the geometry and the constants.  Blocks are 64 x 4.
+// cases, reading each case's x-sweep descriptor: the primitive set the stage
+// reads, the geometry and the constants.
 template <class R, class S>
 __global__ __launch_bounds__(256) void k_les_mut_batch(const SweepArgs<R, S>* __restrict__ cases,
                                                        const TileMap* __restrict__ map, int ncase, int ntiles) {
+  __shared__ LesPlanes<R> pl;
   for (int t = xcd_tile(blockIdx.x, gridDim.x); t < ntiles; t += gridDim.x) {
     const int ci = find_case(map, ncase, t);
     const int local = t - map[ci].start, nbx = map[ci].nbx, nby = map[ci].nby;
     const SweepArgs<R, S>& a = cases[ci];
-    const int i = 1 + (local % nbx) * 64 + (int)threadIdx.x;
-    const int j = 1 + ((local / nbx) % nby) * 4 + (int)threadIdx.y;
-    const int k = 1 + local / (nbx * nby);
-    if (i <= a.g.nx - 2 && j <= a.g.ny - 2) les_mut_cell<S, R>(a.P, a.g, a.c, i, j, k);
-  }
-}
-
-// Persistent batched ghost copy of nu_t and qc2, one pass (tile = 256 items).
-// Blocks are 256 x 1.
-template <class R, class S>
-__global__ __launch_bounds__(256) void k_les_bc_batch(const SweepArgs<R, S>* __restrict__ cases,
-                                                      const TileMap* __restrict__ map, int ncase, int ntiles,
-                                                      int pass) {
-  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const int ci = find_case(map, ncase, t);
-    les_bc_item<S>(cases[ci].P, cases[ci].g, pass, (long long)(t - map[ci].start) * 256 + threadIdx.x);
+    les_mut_tile<S, R>(a.P, a.g, a.c, local % nbx, (local / nbx) % nby, local / (nbx * nby), pl);
+    __syncthreads();  // the next tile overwrites the planes
   }
 }
 

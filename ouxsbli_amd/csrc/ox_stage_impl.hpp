@@ -53,10 +53,9 @@ void prepare_stage(Core& C, const double* Qsrc) {
     prof_mark(C, "prim");
   }
   if constexpr (VISC == 2) {
-    const PhysC<R> cr = make_physc<R>(C.hc);
-    k_les_mut<S, R><<<dim3(cdiv(g.nx - 2, 64), cdiv(g.ny - 2, 4), g.nz - 2), blk, 0, C.stream>>>(P, g, cr);
-    k_les_bc<S><<<(unsigned)((les_bc_items(g, 0) + 255) / 256), 256, 0, C.stream>>>(P, g, 0);
-    k_les_bc<S><<<(unsigned)((les_bc_items(g, 1) + 255) / 256), 256, 0, C.stream>>>(P, g, 1);
+    int bx, by, bz;
+    les_tiles(g, bx, by, bz);
+    k_les_mut<S, R><<<(unsigned)(bx * by * bz), 256, 0, C.stream>>>(P, g, make_physc<R>(C.hc), bx, by);
     prof_mark(C, "les_mut");
   }
 }
@@ -123,17 +122,13 @@ void run_stage(Core& C, const double* Qsrc, const StageArgs& sa, double cx, doub
 }
 
 // One stage of a group of cases: three persistent launches (LES: the SGS
-// viscosity and its two ghost-copy passes first, as in prepare_stage).
+// viscosity first, as in prepare_stage).
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 void run_stage_batch(const BatchGroupLaunch& L) {
   const dim3 blk(64, 4, 1);
   using A = SweepArgs<R, S>;
   if constexpr (VISC == 2) {
-    k_les_mut_batch<R, S><<<L.grid_les[0], blk, 0, L.stream>>>((const A*)L.args[0], L.map_les[0], L.ncase,
-                                                                L.ntiles_les[0]);
-    for (int pass = 0; pass < 2; ++pass)
-      k_les_bc_batch<R, S><<<L.grid_les[1 + pass], 256, 0, L.stream>>>((const A*)L.args[0], L.map_les[1 + pass],
-                                                                        L.ncase, L.ntiles_les[1 + pass], pass);
+    k_les_mut_batch<R, S><<<L.grid_les, 256, 0, L.stream>>>((const A*)L.args[0], L.map_les, L.ncase, L.ntiles_les);
   }
   k_sweep_x_batch<R, S, ORDER, SCHEME, VISC, VO>
       <<<L.grid[0], blk, 0, L.stream>>>((const A*)L.args[0], L.map[0], L.ncase, L.ntiles[0]);
