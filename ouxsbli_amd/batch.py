@@ -12,6 +12,7 @@ HBM budget) and leave when their step count is reached (``done`` /
 from __future__ import annotations
 
 import ctypes
+import threading
 from typing import Optional
 
 import numpy as np
@@ -41,35 +42,50 @@ class PinnedPool:
     ``array(shape)`` returns a float64 numpy array on a pinned buffer; when
     the array (and every view of it) is gone, the buffer goes back to the
     pool for the next result of the same size, up to ``keep_bytes`` retained
-    in all; beyond that it is freed."""
+    in all; beyond that it is freed.  Results beyond ``out_bytes`` held by the
+    program at a time, or that cannot be page-locked, are ordinary arrays.
+    May be used from several threads."""
 
-    def __init__(self, keep_bytes: int = 8 << 30):
+    def __init__(self, keep_bytes: int = 8 << 30, out_bytes: int = 32 << 30):
         self._lib = _native.load()
+        self._lock = threading.RLock()  # a buffer may come back (a finaliser) while it is held
         self._free = {}
         self._kept = 0
+        self._out = 0
         self.keep_bytes = keep_bytes
+        self.out_bytes = out_bytes
 
     def array(self, shape) -> np.ndarray:
         n = int(np.prod(shape))
         nbytes = 8 * n
-        stack = self._free.get(nbytes)
-        if stack:
-            ptr = stack.pop()
-            self._kept -= nbytes
-        else:
+        ptr = None
+        with self._lock:
+            if self._out + nbytes > self.out_bytes:
+                return np.empty(shape, dtype=np.float64)
+            self._out += nbytes
+            stack = self._free.get(nbytes)
+            if stack:
+                ptr = stack.pop()
+                self._kept -= nbytes
+        if ptr is None:
             p = ctypes.c_void_p()
-            _native.check(self._lib.ox_host_alloc(nbytes, ctypes.byref(p)))
+            if self._lib.ox_host_alloc(nbytes, ctypes.byref(p)) != _abi.OX_OK:
+                with self._lock:
+                    self._out -= nbytes
+                return np.empty(shape, dtype=np.float64)
             ptr = p.value
         buf = (ctypes.c_double * n).from_address(ptr)
         buf._release = _Release(self, ptr, nbytes)  # returns the buffer when the last view is gone
         return np.frombuffer(buf, dtype=np.float64).reshape(shape)
 
     def _give_back(self, ptr: int, nbytes: int) -> None:
-        if self._kept + nbytes <= self.keep_bytes:
-            self._free.setdefault(nbytes, []).append(ptr)
-            self._kept += nbytes
-        else:
-            self._lib.ox_host_free(ctypes.c_void_p(ptr))
+        with self._lock:
+            self._out -= nbytes
+            if self._kept + nbytes <= self.keep_bytes:
+                self._free.setdefault(nbytes, []).append(ptr)
+                self._kept += nbytes
+                return
+        self._lib.ox_host_free(ctypes.c_void_p(ptr))
 
 
 class _Release:
@@ -86,14 +102,16 @@ class _Release:
 
 
 _POOL: Optional[PinnedPool] = None
+_POOL_LOCK = threading.Lock()
 
 
 def pinned_pool() -> PinnedPool:
     """The process's pool of pinned result buffers."""
     global _POOL
-    if _POOL is None:
-        _POOL = PinnedPool()
-    return _POOL
+    with _POOL_LOCK:
+        if _POOL is None:
+            _POOL = PinnedPool()
+        return _POOL
 
 
 class Batch:

@@ -16,6 +16,14 @@
 #include "ox2d_core.hpp"
 #include "ox_solver.hpp"
 
+namespace ox2 {
+// dst = src / J (divide) or J * src over n values; dst may be src.
+__global__ __launch_bounds__(256) void k2d_scale(const double* src, double* dst, size_t n, double J, int divide) {
+  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (t < n) dst[t] = divide ? src[t] / J : J * src[t];
+}
+}  // namespace ox2
+
 namespace {
 
 int validate2(const ox2d_config& c) {
@@ -61,16 +69,16 @@ void ox2d_destroy(ox2d_solver* s) {
   if (!s) return;
   hipSetDevice(s->cfg.device);
   if (s->stream) hipStreamSynchronize(s->stream);
-  for (double* b : s->buf)
-    if (b) hipFree(b);
-  if (s->d_args) hipFree(s->d_args);
+  if (s->slab) hipFree(s->slab);
   if (s->ev0) hipEventDestroy(s->ev0);
   if (s->ev1) hipEventDestroy(s->ev1);
   if (s->own_stream) hipStreamDestroy(s->own_stream);
   delete s;
 }
 
-int ox2d_create(const ox2d_config* cfg, ox2d_solver** out) {
+}  // extern "C"
+
+int solver2d_create(const ox2d_config* cfg, hipStream_t shared, ox2d_solver** out) {
   if (!cfg || !out) return ox_fail(OX_EINVAL, "null argument");
   *out = nullptr;
   int rc = validate2(*cfg);
@@ -94,17 +102,16 @@ int ox2d_create(const ox2d_config* cfg, ox2d_solver** out) {
     return ox_fail(code, msg);
   };
   if (hipSetDevice(cfg->device) != hipSuccess) return fail(OX_EDEVICE, "hipSetDevice failed");
-  if (hipStreamCreateWithFlags(&s->own_stream, hipStreamNonBlocking) != hipSuccess ||
+  if ((!shared && hipStreamCreateWithFlags(&s->own_stream, hipStreamNonBlocking) != hipSuccess) ||
       hipEventCreate(&s->ev0) != hipSuccess || hipEventCreate(&s->ev1) != hipSuccess)
     return fail(OX_EDEVICE, "stream/event creation failed");
-  s->stream = s->own_stream;
-  const size_t bytes = state2_elems(*cfg) * sizeof(double);
-  for (double*& b : s->buf) {
-    if (hipMalloc(&b, bytes) != hipSuccess) return fail(OX_ENOMEM, "device allocation failed");
-    if (hipMemsetAsync(b, 0, bytes, s->stream) != hipSuccess) return fail(OX_EDEVICE, "hipMemsetAsync failed");
-  }
+  s->stream = shared ? shared : s->own_stream;
+  const size_t bytes = (state2_elems(*cfg) * sizeof(double) + 255) & ~(size_t)255;
   s->args_bytes = ox2::args2_bytes(cfg->precision);
-  if (hipMalloc(&s->d_args, 3 * s->args_bytes) != hipSuccess) return fail(OX_ENOMEM, "device allocation failed");
+  if (hipMalloc(&s->slab, 3 * bytes + 3 * s->args_bytes) != hipSuccess) return fail(OX_ENOMEM, "device allocation failed");
+  if (hipMemsetAsync(s->slab, 0, 3 * bytes, s->stream) != hipSuccess) return fail(OX_EDEVICE, "hipMemsetAsync failed");
+  for (int k = 0; k < 3; ++k) s->buf[k] = (double*)(s->slab + k * bytes);
+  s->d_args = s->slab + 3 * bytes;
   std::vector<char> h(3 * s->args_bytes);
   for (int st = 0; st < 3; ++st) ox2::write_args2(*cfg, s->g, s->buf, st, 0, h.data() + st * s->args_bytes);
   if (hipMemcpyAsync(s->d_args, h.data(), h.size(), hipMemcpyHostToDevice, s->stream) != hipSuccess ||
@@ -117,14 +124,18 @@ int ox2d_create(const ox2d_config* cfg, ox2d_solver** out) {
   return OX_OK;
 }
 
+extern "C" {
+
+int ox2d_create(const ox2d_config* cfg, ox2d_solver** out) { return solver2d_create(cfg, nullptr, out); }
+
 int ox2d_set_state(ox2d_solver* s, const double* Q) {
   if (!s || !Q) return ox_fail(OX_EINVAL, "null argument");
   OX_HIP(hipSetDevice(s->cfg.device));
   const size_t n = state2_elems(s->cfg);
-  std::vector<double> qj(n);
-  const double J = s->g.J;
-  for (size_t t = 0; t < n; ++t) qj[t] = Q[t] / J;  // pre_calc: QJ = Q / J
-  OX_HIP(hipMemcpyAsync(s->buf[0], qj.data(), n * sizeof(double), hipMemcpyHostToDevice, s->stream));
+  OX_HIP(hipMemcpyAsync(s->buf[0], Q, n * sizeof(double), hipMemcpyHostToDevice, s->stream));
+  // pre_calc: QJ = Q / J
+  ox2::k2d_scale<<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->buf[0], s->buf[0], n, s->g.J, 1);
+  OX_HIP(hipGetLastError());
   OX_HIP(hipStreamSynchronize(s->stream));
   return OX_OK;
 }
@@ -133,10 +144,12 @@ int ox2d_get_state(ox2d_solver* s, double* Q) {
   if (!s || !Q) return ox_fail(OX_EINVAL, "null argument");
   OX_HIP(hipSetDevice(s->cfg.device));
   const size_t n = state2_elems(s->cfg);
-  OX_HIP(hipMemcpyAsync(Q, s->buf[0], n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+  // main.f90:84: Q = J * QJ, into the first stage's buffer, which holds no live
+  // data between steps (every stage writes all points of its output)
+  ox2::k2d_scale<<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->buf[0], s->buf[1], n, s->g.J, 0);
+  OX_HIP(hipGetLastError());
+  OX_HIP(hipMemcpyAsync(Q, s->buf[1], n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
   OX_HIP(hipStreamSynchronize(s->stream));
-  const double J = s->g.J;
-  for (size_t t = 0; t < n; ++t) Q[t] = J * Q[t];  // main.f90:84: Q = J * QJ
   return OX_OK;
 }
 

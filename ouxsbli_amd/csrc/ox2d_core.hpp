@@ -141,6 +141,7 @@ inline int grid2(int ntiles, int cap) {
 struct ox2d_solver {
   ox2d_config cfg{};
   ox2::Geom2 g{};
+  char* slab = nullptr;                          // the device memory of the arrays below
   double* buf[3] = {nullptr, nullptr, nullptr};  // A = Q^n, B, C
   char* d_args = nullptr;                          // the three stage descriptors
   size_t args_bytes = 0;
@@ -152,3 +153,5 @@ struct ox2d_solver {
 };
 
 size_t solver2d_footprint(const ox2d_config& c);
+// ox2d_create on `shared` instead of a stream of the handle's own (null: its own).
+int solver2d_create(const ox2d_config* cfg, hipStream_t shared, ox2d_solver** out);

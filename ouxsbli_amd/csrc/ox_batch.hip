@@ -38,7 +38,6 @@ void ox_destroy(ox_solver* s);
 int ox_set_state(ox_solver* s, const double* Q);
 int ox_get_state(ox_solver* s, double* Q);
 int ox_autotune(ox_solver* s, int32_t* lseg_y, int32_t* lseg_z);
-int ox2d_create(const ox2d_config* cfg, ox2d_solver** out);
 void ox2d_destroy(ox2d_solver* s);
 int ox2d_set_state(ox2d_solver* s, const double* Q);
 int ox2d_get_state(ox2d_solver* s, double* Q);
@@ -445,15 +444,9 @@ void enqueue_step(ox_batch* b, int set) {
   }
 }
 
-// Returns a case's solver to its own stream and frees it.
 void free_case(BCase* c) {
-  if (c->s2) {
-    c->s2->stream = c->s2->own_stream;
-    ox2d_destroy(c->s2);
-  } else {
-    c->s->C.stream = c->s->own_stream;
-    ox_destroy(c->s);
-  }
+  if (c->s2) ox2d_destroy(c->s2);
+  else ox_destroy(c->s);
 }
 
 }  // namespace
@@ -472,7 +465,7 @@ int admit3d(ox_batch* b, const ox_config* cfg, Init init, int32_t nsteps, int64_
   if ((int)(b->active.size() + b->done.size()) >= b->cfg.max_cases) return ox_fail(OX_EBUSY, "no free slot");
   if (b->bytes_in_use + need > b->cfg.hbm_budget) return ox_fail(OX_EBUSY, "footprint exceeds the free HBM budget");
   ox_solver* s = nullptr;
-  int rc = ox_create(cfg, &s);
+  int rc = solver_create(cfg, b->stream, &s);
   if (rc != OX_OK) return rc;
   rc = init(s);
   if (rc == OX_OK && b->cfg.autotune) rc = tune_case(b, s);
@@ -480,8 +473,7 @@ int admit3d(ox_batch* b, const ox_config* cfg, Init init, int32_t nsteps, int64_
     ox_destroy(s);
     return rc;
   }
-  // primitives of the initial state on the handle's own stream, then the
-  // case joins the engine's stream
+  // primitives of the initial state
   {
     ox::BatchOps ops;
     const bool ok = cfg->precision == OX_PREC_FP64
@@ -497,7 +489,6 @@ int admit3d(ox_batch* b, const ox_config* cfg, Init init, int32_t nsteps, int64_
       return ox_fail(OX_EDEVICE, "case initialisation failed");
     }
   }
-  s->C.stream = b->stream;
   s->C.prof = false;
   auto c = std::make_unique<BCase>();
   c->id = b->next_id++;
@@ -644,14 +635,13 @@ int ox_batch_admit2d(ox_batch* b, const ox2d_config* cfg, const double* Q, int32
   if ((int)(b->active.size() + b->done.size()) >= b->cfg.max_cases) return ox_fail(OX_EBUSY, "no free slot");
   if (b->bytes_in_use + need > b->cfg.hbm_budget) return ox_fail(OX_EBUSY, "footprint exceeds the free HBM budget");
   ox2d_solver* s = nullptr;
-  int rc = ox2d_create(cfg, &s);
+  int rc = solver2d_create(cfg, b->stream, &s);
   if (rc != OX_OK) return rc;
   rc = Q ? ox2d_set_state(s, Q) : ox2d_init_state(s);
   if (rc != OX_OK) {
     ox2d_destroy(s);
     return rc;
   }
-  s->stream = b->stream;
   auto c = std::make_unique<BCase>();
   c->id = b->next_id++;
   c->s2 = s;

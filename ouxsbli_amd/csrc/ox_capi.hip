@@ -280,13 +280,7 @@ ox::Geom make_geom(const ox_config& c) {
 
 void destroy(ox_solver* s) {
   if (!s) return;
-  hipFree(s->QJ);
-  hipFree(s->QJ2);
-  hipFree(s->Rs);
-  hipFree(s->scratch);
-  hipFree(s->C.Racc);
-  for (int set = 0; set < 2; ++set)
-    for (int m = 0; m < ox::kPrimArrays; ++m) hipFree(s->C.prim[set][m]);
+  hipFree(s->slab);
   for (hipEvent_t e : s->prof.pool) hipEventDestroy(e);
   if (s->ev0) hipEventDestroy(s->ev0);
   if (s->ev1) hipEventDestroy(s->ev1);
@@ -336,36 +330,7 @@ void launch_ghost_fill(Core& C, double* Q) {
 }
 }  // namespace ox
 
-extern "C" {
-
-const char* ox_last_error(void) { return g_err.c_str(); }
-
-int ox_host_alloc(uint64_t bytes, void** ptr) {
-  if (!ptr || bytes == 0) return ox_fail(OX_EINVAL, "null pointer or zero size");
-  *ptr = nullptr;
-  OX_HIP(hipHostMalloc(ptr, (size_t)bytes, hipHostMallocDefault));
-  return OX_OK;
-}
-
-int ox_host_free(void* ptr) {
-  if (!ptr) return OX_OK;
-  OX_HIP(hipHostFree(ptr));
-  return OX_OK;
-}
-
-const char* ox_version(void) { return "ouxsbli-mi355x 1 gfx950"; }
-
-int ox_real4_sum(const double* terms, int64_t n, float* out) {
-  if (!out || (n > 0 && !terms) || n < 0) return ox_fail(OX_EINVAL, "null argument or negative count");
-  // a REAL(4) accumulator: each REAL(8) term is added in double precision and
-  // the sum rounded back to single, in order
-  float acc = 0.0f;
-  for (int64_t m = 0; m < n; ++m) acc = (float)((double)acc + terms[m]);
-  *out = acc;
-  return OX_OK;
-}
-
-int ox_create(const ox_config* cfg, ox_solver** out) {
+int solver_create(const ox_config* cfg, hipStream_t shared, ox_solver** out) {
   if (!cfg || !out) return ox_fail(OX_EINVAL, "null argument");
   *out = nullptr;
   int rc = validate(*cfg);
@@ -421,32 +386,39 @@ int ox_create(const ox_config* cfg, ox_solver** out) {
   ox::solo_segments(C.g, ops, C.lseg);
   const size_t ns = state_elems(C.g), nc = cell_elems(C.g);
   const size_t pe = cfg->precision == OX_PREC_FP64 ? sizeof(double) : sizeof(float);
-  bool ok = hipStreamCreateWithFlags(&C.stream, hipStreamNonBlocking) == hipSuccess;
-  s->own_stream = C.stream;
-  ok = ok && hipMalloc(&s->QJ, ns * sizeof(double)) == hipSuccess;
-  ok = ok && hipMalloc(&s->QJ2, ns * sizeof(double)) == hipSuccess;
-  ok = ok && hipMalloc(&C.Racc, ns * pe) == hipSuccess;
-  if (cfg->rk == 4) ok = ok && hipMalloc(&s->Rs, ns * sizeof(double)) == hipSuccess;
-  // arrays 6 and 7 (mut, qc2) only for LES
-  const int nprim = cfg->visc == OX_VISC_LES ? 8 : 6;
-  for (int set = 0; set < 2; ++set)
-    for (int m = 0; m < nprim && ok; ++m)
-      ok = hipMalloc(&C.prim[set][m], nc * pe) == hipSuccess;
+  bool ok = shared || hipStreamCreateWithFlags(&s->own_stream, hipStreamNonBlocking) == hipSuccess;
+  C.stream = shared ? shared : s->own_stream;
+  // every array of the handle in one allocation: a hipFree of more than a few
+  // MB costs about 0.1 ms, whatever its size
+  const int nprim = cfg->visc == OX_VISC_LES ? 8 : 6;  // arrays 6 and 7 (mut, qc2) only for LES
   s->scratch_bytes = 4096 * (2 * ox::DIAG_NQ + 1) * sizeof(double);
-  ok = ok && hipMalloc(&s->scratch, s->scratch_bytes) == hipSuccess;
+  size_t bytes = 0;
+  auto place = [&bytes](size_t n) {
+    const size_t at = bytes;
+    bytes += (n + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t at_qj = place(ns * sizeof(double)), at_qj2 = place(ns * sizeof(double)), at_racc = place(ns * pe);
+  const size_t at_rs = cfg->rk == 4 ? place(ns * sizeof(double)) : 0;
+  size_t at_prim[2][8];
+  for (int set = 0; set < 2; ++set)
+    for (int m = 0; m < nprim; ++m) at_prim[set][m] = place(nc * pe);
+  const size_t cleared = bytes, at_scratch = place(s->scratch_bytes);
+  ok = ok && hipMalloc(&s->slab, bytes) == hipSuccess;
   ok = ok && hipEventCreate(&s->ev0) == hipSuccess && hipEventCreate(&s->ev1) == hipSuccess;
   if (!ok) {
     destroy(s);
     return ox_fail(OX_ENOMEM, "device allocation failed");
   }
-  // Zero everything once: ghost layers of QJ2 and the accumulators start defined.
-  ok = hipMemsetAsync(s->QJ, 0, ns * sizeof(double), C.stream) == hipSuccess;
-  ok = ok && hipMemsetAsync(s->QJ2, 0, ns * sizeof(double), C.stream) == hipSuccess;
-  ok = ok && hipMemsetAsync(C.Racc, 0, ns * pe, C.stream) == hipSuccess;
-  if (s->Rs) ok = ok && hipMemsetAsync(s->Rs, 0, ns * sizeof(double), C.stream) == hipSuccess;
+  s->QJ = (double*)(s->slab + at_qj);
+  s->QJ2 = (double*)(s->slab + at_qj2);
+  C.Racc = s->slab + at_racc;
+  if (cfg->rk == 4) s->Rs = (double*)(s->slab + at_rs);
   for (int set = 0; set < 2; ++set)
-    for (int m = 0; m < nprim && ok; ++m)
-      ok = hipMemsetAsync(C.prim[set][m], 0, nc * pe, C.stream) == hipSuccess;
+    for (int m = 0; m < nprim; ++m) C.prim[set][m] = s->slab + at_prim[set][m];
+  s->scratch = (double*)(s->slab + at_scratch);
+  // Zero everything once: ghost layers of QJ2 and the accumulators start defined.
+  ok = hipMemsetAsync(s->slab, 0, cleared, C.stream) == hipSuccess;
   ok = ok && hipStreamSynchronize(C.stream) == hipSuccess;
   if (!ok) {
     destroy(s);
@@ -455,6 +427,37 @@ int ox_create(const ox_config* cfg, ox_solver** out) {
   *out = s;
   return OX_OK;
 }
+
+extern "C" {
+
+const char* ox_last_error(void) { return g_err.c_str(); }
+
+int ox_host_alloc(uint64_t bytes, void** ptr) {
+  if (!ptr || bytes == 0) return ox_fail(OX_EINVAL, "null pointer or zero size");
+  *ptr = nullptr;
+  OX_HIP(hipHostMalloc(ptr, (size_t)bytes, hipHostMallocDefault));
+  return OX_OK;
+}
+
+int ox_host_free(void* ptr) {
+  if (!ptr) return OX_OK;
+  OX_HIP(hipHostFree(ptr));
+  return OX_OK;
+}
+
+const char* ox_version(void) { return "ouxsbli-mi355x 1 gfx950"; }
+
+int ox_real4_sum(const double* terms, int64_t n, float* out) {
+  if (!out || (n > 0 && !terms) || n < 0) return ox_fail(OX_EINVAL, "null argument or negative count");
+  // a REAL(4) accumulator: each REAL(8) term is added in double precision and
+  // the sum rounded back to single, in order
+  float acc = 0.0f;
+  for (int64_t m = 0; m < n; ++m) acc = (float)((double)acc + terms[m]);
+  *out = acc;
+  return OX_OK;
+}
+
+int ox_create(const ox_config* cfg, ox_solver** out) { return solver_create(cfg, nullptr, out); }
 
 void ox_destroy(ox_solver* s) {
   if (!s) return;

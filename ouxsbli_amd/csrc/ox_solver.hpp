@@ -22,6 +22,7 @@ struct ProfState {
 struct ox_solver {
   ox::Core C;
   ProfState prof;
+  char* slab = nullptr;   // the device memory of every array below and of the Core
   double* QJ = nullptr;   // state Q^n
   double* QJ2 = nullptr;  // QJ2 (RK3) / QJs (RK4)
   double* Rs = nullptr;   // RK4 accumulator
@@ -50,6 +51,11 @@ void prof_record(ox::Core* C, const char* name);
 // Stage `st` (0-based) of one RK step of handle s: source state, epilogue and
 // the factor on dt * face area.
 void rk_stage(ox_solver* s, int st, const double** Qsrc, ox::StageArgs* sa, double* coef);
+
+// ox_create on `shared` instead of a stream of the handle's own (null: its own).
+// The batch engine's cases run on its stream and own none: every hipFree waits on
+// each stream of the process, which made retiring one of 64 cases take 0.9 ms.
+int solver_create(const ox_config* cfg, hipStream_t shared, ox_solver** out);
 
 // Device bytes a handle with this configuration allocates.
 size_t solver_footprint(const ox_config& c);
