@@ -236,7 +236,7 @@ int build_plan(ox_batch* b) {
         ox::TileMap m{};
         unsigned nbx, nby, nbz;
         if (d == 0) {
-          nbx = cdivu(g.ix, G.ops.xt); nby = cdivu(g.iy, ox::XROWS); nbz = g.iz;
+          nbx = (unsigned)ox::xrun_blocks(g); nby = nbz = 1;
         } else if (d == 1) {
           nbx = ox::line_tiles(g, 1); nby = 1; nbz = cdivu(g.iy, ls[0]);
         } else {
@@ -286,7 +286,8 @@ int build_plan(ox_batch* b) {
         for (int d = 0; d < 3; ++d) {
           L.map[d] = b->d_map + map_off[gi] + (size_t)d * n;
           L.ntiles[d] = ntiles[gi][d];
-          L.grid[d] = std::max(1, std::min(ntiles[gi][d], kMaxGrid));
+          // the x sweep takes one workgroup per run
+          L.grid[d] = d == 0 ? ntiles[gi][0] : std::max(1, std::min(ntiles[gi][d], kMaxGrid));
         }
         if (G.les) {
           L.map_les = b->d_map + map_off[gi] + (size_t)3 * n;

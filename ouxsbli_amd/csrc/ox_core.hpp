@@ -91,7 +91,6 @@ struct BatchGroupLaunch {
 
 struct BatchOps {
   size_t args_bytes;  // size of one sweep descriptor
-  int xt;             // interior cells per x tile
   // k_prim when the primitives are stale; the LES viscosity of the stage
   void (*prepare)(Core& C, const double* Qsrc);
   // the three sweep descriptors (x, y, z) of one case for one stage

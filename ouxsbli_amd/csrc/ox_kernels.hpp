@@ -9,8 +9,9 @@
 //          formed from rho and p where a sweep reads a cell.
 //   Racc   residual accumulator in the state layout, type S.
 //
-// One stage = k_sweep_x (LDS row tiles; Ducros sensor; writes R = c_x*dE; on
-// periodic rows of 64, 128 or 256 cells k_sweep_xrow, whole rows in LDS) -> k_sweep_line<DIR=1>
+// One stage = k_sweep_x (runs of faces in LDS rows; Ducros sensor; writes
+// R = c_x*dE; on periodic rows of 64, 128 or 256 cells k_sweep_xrow, whole rows
+// in LDS) -> k_sweep_line<DIR=1>
 // (register sliding window along y; R += c_y*dF) -> k_sweep_line<DIR=2>
 // (sliding window along z; R += c_z*dG, then the RK combination, and the
 // primitives of the new state for the next stage).  k_prim (QJ -> primitives)
@@ -77,9 +78,6 @@ template <int ORDER, int VISC, int VO> struct Sten {
 // two.  The map is a permutation of [0, n).
 #ifndef OX_XCD_SWIZZLE
 #define OX_XCD_SWIZZLE 1
-#endif
-#ifndef OX_XSWEEP_ZMAJOR
-#define OX_XSWEEP_ZMAJOR 1
 #endif
 __device__ __forceinline__ int xcd_tile(int b, int n) {
   if (!OX_XCD_SWIZZLE || (n & 7)) return b;
@@ -392,23 +390,41 @@ __device__ __forceinline__ void cross_fields(const Prim<S>& P, const Geom& g, co
   }
 }
 
+// A cell by its index (the line sweeps), or as the x sweep's waves address it: an
+// index that is the same for all lanes, kept in scalar registers, and this lane's
+// distance from it in bytes.  The second form leaves a load's address to the
+// scalar unit: 115 vector instructions less in the FP64 SLAU6 NS run, and 437 ->
+// 415 us for Hybrid6 LES 192^3.  In the line sweeps' loops it spilled scalar
+// registers.
+struct CellAt {
+  long long u;
+  unsigned lane;
+};
+template <class S> __device__ __forceinline__ S at(const S* f, const CellAt& c, long long off = 0) {
+  using GC = __attribute__((address_space(1))) const char;
+  using GS = __attribute__((address_space(1))) const S;
+  return *(GS*)((GC*)G(f + (c.u + off)) + c.lane);
+}
+template <class S> __device__ __forceinline__ S at(const S* f, int m, int off = 0) { return G(f)[m + off]; }
+
 // Issues the loads of cell m (sensor read at ms, its periodic image): its own
 // values, and the transverse stencil values of a viscous run.
-template <class S, int DIR, int ORDER, int SCHEME, int VISC, int VO, bool LOAD_S = true>
-__device__ __forceinline__ void fetch_values(const Prim<S>& P, int m, int ms, RawCell<S, VISC, VO>& r) {
-  r.rho = G(P.rho)[m];
-  r.u = G(P.u)[m];
-  r.v = G(P.v)[m];
-  r.w = G(P.w)[m];
-  r.p = G(P.p)[m];
-  if constexpr (LOAD_S && kUsesSensor<SCHEME, ORDER>) r.s = G(P.s)[ms];
+template <class S, int DIR, int ORDER, int SCHEME, int VISC, int VO, bool LOAD_S = true, class C>
+__device__ __forceinline__ void fetch_values(const Prim<S>& P, const C& m, const C& ms,
+                                             RawCell<S, VISC, VO>& r) {
+  r.rho = at(P.rho, m);
+  r.u = at(P.u, m);
+  r.v = at(P.v, m);
+  r.w = at(P.w, m);
+  r.p = at(P.p, m);
+  if constexpr (LOAD_S && kUsesSensor<SCHEME, ORDER>) r.s = at(P.s, ms);
   if constexpr (VISC == 2) {
-    r.mt = G(P.mut)[m];
-    r.qc2 = G(P.qc2)[m];
+    r.mt = at(P.mut, m);
+    r.qc2 = at(P.qc2, m);
   }
 }
-template <class S, int DIR, int VISC, int VO>
-__device__ __forceinline__ void fetch_cross(const Prim<S>& P, const Geom& g, int m, RawCell<S, VISC, VO>& r) {
+template <class S, int DIR, int VISC, int VO, class C>
+__device__ __forceinline__ void fetch_cross(const Prim<S>& P, const Geom& g, const C& m, RawCell<S, VISC, VO>& r) {
   if constexpr (VISC) {
     const S* f[4];
     int st[4];
@@ -419,13 +435,14 @@ __device__ __forceinline__ void fetch_cross(const Prim<S>& P, const Geom& g, int
 #pragma unroll
       for (int t = 0; t < VC; ++t) {
         const int off = t < VC / 2 ? t - VC / 2 : t - VC / 2 + 1;
-        r.x[q][t] = G(f[q])[m + off * st[q]];
+        r.x[q][t] = at(f[q], m, off * st[q]);
       }
     }
   }
 }
-template <class S, int DIR, int ORDER, int SCHEME, int VISC, int VO, bool LOAD_S = true>
-__device__ __forceinline__ void fetch_cell(const Prim<S>& P, const Geom& g, int m, int ms, RawCell<S, VISC, VO>& r) {
+template <class S, int DIR, int ORDER, int SCHEME, int VISC, int VO, bool LOAD_S = true, class C>
+__device__ __forceinline__ void fetch_cell(const Prim<S>& P, const Geom& g, const C& m, const C& ms,
+                                           RawCell<S, VISC, VO>& r) {
   fetch_values<S, DIR, ORDER, SCHEME, VISC, VO, LOAD_S>(P, m, ms, r);
   fetch_cross<S, DIR, VISC, VO>(P, g, m, r);
 }
@@ -567,6 +584,7 @@ template <class R, class S> struct SweepArgs {
   double cd;        // c_x, c_y or c_z of calc_R (stage coefficient * dt * face area)
   int tvd, variant;
   int lseg;         // cells per thread segment in the y / z sweeps
+  int xrows, xwgs;  // x sweep: rows of a band, workgroups per band and plane
 };
 
 struct TileMap {
@@ -574,25 +592,6 @@ struct TileMap {
   int nbx, nby;  // tiles along the three launch dimensions
   int nbz;
 };
-
-// The x sweep's tiles (bx, row band by, plane bz) in x, z, y order under
-// xcd_tile: one XCD's run covers a band of rows through many planes, so both
-// the y and the z neighbours a row tile's cross-derivative stencils read
-// (rows by +- 1, planes bz +- 3) are fetched by tiles resident at about the
-// same time in one L2.
-__device__ __forceinline__ void launch_tile_xzy(int& bx, int& by, int& bz) {
-  const int gx = gridDim.x, gy = gridDim.y, gz = gridDim.z;
-  const int t = xcd_tile(blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z), gx * gy * gz);
-#if OX_XSWEEP_ZMAJOR
-  bx = t % gx;
-  bz = (t / gx) % gz;
-  by = t / (gx * gz);
-#else
-  bx = t % gx;
-  by = (t / gx) % gy;
-  bz = t / (gx * gy);
-#endif
-}
 
 // Case owning global tile t (map[].start ascending, map[0].start == 0).
 __device__ __forceinline__ int find_case(const TileMap* __restrict__ map, int ncase, int t) {
@@ -605,18 +604,9 @@ __device__ __forceinline__ int find_case(const TileMap* __restrict__ map, int nc
   return lo;
 }
 
-// ---------------------------------------------------------------------------
-// x sweep.  One wavefront per grid row: the tile of a row is exactly 64 cells
-// wide (XT = 64 - SW interior cells plus the stencil halo), so every lane
-// loads one cell, and lanes 0..XT compute the XT+1 faces the interior cells
-// need; the right-face flux of each cell comes from the neighbouring lane by
-// a cross-lane shuffle.
-// ---------------------------------------------------------------------------
 #ifndef OX_SPLIT_FENCE
 #define OX_SPLIT_FENCE() asm volatile("" ::: "memory")
 #endif
-template <int ORDER, int VISC, int VO> constexpr int xtile() { return 64 - Sten<ORDER, VISC, VO>::SW; }
-constexpr int XROWS = 4;
 
 // Ducros sensor of one cell (calc_Ducros, 3D_solver/src/calc_hybrid.f90:11-72)
 // from its six face neighbours' velocities.
@@ -678,170 +668,257 @@ __device__ __forceinline__ R ducros_x(const Geom& g, const DucrosPart<R>& d, R u
   return fmin2(R(1), fd);
 }
 
+// ---------------------------------------------------------------------------
+// x sweep: runs of faces.  A row of ix cells has ix + 1 faces; the faces of a
+// band of rows of one plane, row after row, are dealt to waves, one face per
+// lane, each starting at the last face of the wave before (its first cell needs
+// that face too); the four waves of a workgroup share the LDS rows.  A lane
+// loads the cell right of its face; the SW - 1 other cells that the faces of a
+// row piece read, left and right of it, are loaded by the first lanes.  The LDS
+// rows are structure-of-arrays so that lane-consecutive reads are bank-conflict
+// free.  The flux of a cell's right face comes from the next lane.
+//
 // Writes Racc = c_x * (E_right - E_left) (the first term of calc_R).  For
 // the schemes that read the Ducros sensor the sweep also computes it for its
-// row and stores it for the y and z sweeps.  The LDS tile is
-// structure-of-arrays so that lane-consecutive reads are bank-conflict free.
-template <int VISC> constexpr int xsweep_nf() { return VISC == 2 ? 14 : 12; }  // rho,u,v,w,p,T,mu,s,d1..d4[,mt,H]
+// cells and stores it for the y and z sweeps.
+//
+// Bound by the vector units (0.88 busy in FP64), so by the lanes that hold no
+// face.  Row tiles of one wave, 64 less the halo's SW - 1, spent 192 lanes on a
+// row of 124 cells and 128 on one of 80; runs lose one lane in 64, the halo cells'
+// loads and the end of a band.  Measured (us), tiles -> runs: FP64 SLAU6 NS 80 x
+// 112 x 48 38 -> 29, 124^3 122 -> 101, 192^3 417 -> 366; Hybrid6 LES 64^3 35 -> 26,
+// 192^3 494 -> 415, 256^3 1088 -> 958; KEEP4 NS 192^3 241 -> 226, 96^3 23.1 -> 24.8
+// (rows of 97 faces fit two tiles as well, and memory bounds it); FP32 Roe4 NS
+// 124^3 52 -> 44, SLAU6 Euler 124^3 49 -> 41, KEEP4 Euler 144^3 34 -> 30.
+// ---------------------------------------------------------------------------
+// The fields of an LDS row: rho,u,v,w,p, then those that the scheme reads.
+template <int ORDER, int SCHEME, int VISC> struct XFields {
+  static constexpr int T = 5;
+  static constexpr int s = T + (kUsesT<SCHEME> || VISC ? 1 : 0);
+  static constexpr int mu = s + (kUsesSensor<SCHEME, ORDER> ? 1 : 0);
+  static constexpr int d = mu + 1;  // d1..d4
+  static constexpr int mt = d + 4, H = mt + 1;
+  static constexpr int N = VISC == 0 ? mu : VISC == 1 ? mt : H + 1;
+};
+constexpr int XRUN = 4 * 63;  // cells of a run: 64 faces per wave, one shared with the next wave
+// row pieces of a run at most: rows have at least 2 ORDER + 1 faces
+template <int ORDER> constexpr int xrun_pieces() { return XRUN / (2 * ORDER + 1) + 2; }
+template <int ORDER, int VISC, int VO> constexpr int xrun_len() {
+  return XRUN + 1 + (Sten<ORDER, VISC, VO>::SW - 1) * xrun_pieces<ORDER>();
+}
+template <class R, int ORDER, int SCHEME, int VISC, int VO> struct XRunTile {
+  R f[XFields<ORDER, SCHEME, VISC>::N][xrun_len<ORDER, VISC, VO>()];
+};
+
+// Rows per band and workgroups per band and plane: the workgroups of a band walk
+// its planes, so that the y neighbours of the cross-derivative and sensor stencils
+// are read once per band from L2; 8 to 32 rows, the number that leaves the
+// fewest lanes idle, near 16 where several do.
+inline void xrun_shape(const Geom& g, int& rows, int& wgs) {
+  long long best = -1;
+  rows = wgs = 1;
+  for (int d = 0; d <= 24; ++d) {
+    const int n = 16 + ((d & 1) ? (d + 1) / 2 : -(d / 2));  // 16, 17, 15, 18, 14, ...
+    if (n < 8 || n > 32) continue;
+    const int m = n < g.iy ? n : g.iy;
+    const long long per = ((long long)m * (g.ix + 1) - 1 + XRUN - 1) / XRUN;
+    const long long total = per * ((g.iy + m - 1) / m);
+    if (best < 0 || total < best) best = total, rows = m, wgs = (int)per;
+  }
+}
+inline long long xrun_blocks(const Geom& g) {
+  int rows, wgs;
+  xrun_shape(g, rows, wgs);
+  return (long long)wgs * g.iz * ((g.iy + rows - 1) / rows);
+}
 
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
-__device__ __forceinline__ void sweep_x_tile(const SweepArgs<R, S>& a, int bx, int by, int bz,
-                                             R (&tile)[xsweep_nf<VISC>()][XROWS][64]) {
-  const Prim<S>& P = a.P;
-  S* __restrict__ Racc = a.Racc;
-  const Geom& g = a.g;
-  const PhysC<R>& c = a.c;
-  const int tvd = a.tvd, variant = a.variant;
-  const double cx = a.cd;
+__device__ __forceinline__ void sweep_x_run(const SweepArgs<R, S>& a, int t, XRunTile<R, ORDER, SCHEME, VISC, VO>& lds) {
   using St = Sten<ORDER, VISC, VO>;
   using CD = CellData<R, 0, ORDER, SCHEME, VISC, VO>;
   using RC = RawCell<S, VISC, VO>;
   constexpr bool SENS = kUsesSensor<SCHEME, ORDER>;
-  constexpr int XT = xtile<ORDER, VISC, VO>();
-  constexpr int W = XT + St::SW;
-  static_assert(W == 64, "one tile cell per lane");
   // With one ghost layer (ORDER 2) a ghost cell's sensor is the boundary copy
   // of its interior neighbour (calc_hybrid.f90:54-71), taken from a clamped
   // index; with more layers every sensor the faces read belongs to a cell in
-  // 1..nx-2 whose x neighbours are in the row tile.
+  // 1..nx-2 whose x neighbours are in the LDS row.
   constexpr bool SPLIT_SENS = SENS && ORDER > 2;
-  constexpr int NF = xsweep_nf<VISC>();
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const int i0 = g.h + bx * XT;
-  const int j = g.h + by * XROWS + ty;
-  const int k = g.h + bz;
-  const bool rowok = j < g.h + g.iy;
-  const int m = tx;                // this lane's tile position
-  const int i = i0 - St::HW + m;   // and its cell
+  // With few fields and little arithmetic the loads' latency shows: the halo's go
+  // first (FP32 KEEP Euler 144^3 33 -> 30 us; SLAU6 Euler lost 3%).
+  constexpr bool EARLY = SCHEME == KEEP && !VISC;
+  using XF = XFields<ORDER, SCHEME, VISC>;
+  constexpr int HW = St::HW, SW = St::SW;
+  static_assert((SW - 1) * xrun_pieces<ORDER>() <= 256, "one halo cell per lane");
+  auto& tile = lds.f;
+  const Prim<S>& P = a.P;
+  const Geom& g = a.g;
+  const PhysC<R>& c = a.c;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int sy = g.nx, sz = g.nx * g.ny;
-  // sensor positions: the cells either side of the XT+1 faces
-  const bool spos = m >= St::HW - 1 && m <= St::HW + XT && i <= g.nx - 2;
-  DucrosPart<R> dp{};
-  if (rowok && i < g.nx) {
-    const int q = cidx(g, i, j, k);
-    RC r;
-    fetch_cell<S, 0, ORDER, SCHEME, VISC, VO, false>(P, g, q, 0, r);
-    if constexpr (SPLIT_SENS) {
-      if (spos) {
-        constexpr int H = vcross<VO>() / 2;  // r.x[.][H-1], r.x[.][H]: the -1 and +1 neighbours
-        R uym, uyp, vym, vyp, uzm, uzp, wzm, wzp;
-        if constexpr (VISC) {  // DIR 0 cross stencils: u,v along y; u,w along z
-          uym = R(r.x[0][H - 1]); uyp = R(r.x[0][H]);
-          vym = R(r.x[1][H - 1]); vyp = R(r.x[1][H]);
-          uzm = R(r.x[2][H - 1]); uzp = R(r.x[2][H]);
-          wzm = R(r.x[3][H - 1]); wzp = R(r.x[3][H]);
-        } else {
-          uym = R(G(P.u)[q - sy]); uyp = R(G(P.u)[q + sy]);
-          vym = R(G(P.v)[q - sy]); vyp = R(G(P.v)[q + sy]);
-          uzm = R(G(P.u)[q - sz]); uzp = R(G(P.u)[q + sz]);
-          wzm = R(G(P.w)[q - sz]); wzp = R(G(P.w)[q + sz]);
-        }
-        dp = ducros_yz<R>(g, uym, uyp, vym, vyp, R(G(P.w)[q - sy]), R(G(P.w)[q + sy]), uzm, uzp, R(G(P.v)[q - sz]),
-                          R(G(P.v)[q + sz]), wzm, wzp);
-      }
+  // run w of plane k and band of rows j0 ..: faces c0 .. last of the band's rows
+  const int n1 = g.ix + 1;  // faces of a row
+  const int w = t % a.xwgs, kb = t / a.xwgs;
+  const int k = g.h + kb % g.iz, j0 = kb / g.iz * a.xrows;
+  const int total = min(a.xrows, g.iy - j0) * n1;
+  const int c0 = w * XRUN, last = min(XRUN, total - 1 - c0);
+  if (last < 1) return;  // (the whole workgroup) a shorter last band
+  const int p0 = c0 / n1, f0 = c0 - p0 * n1;  // the run's first row and face
+  // piece of lane (or face offset) x: rows shorter than a run by an exact float
+  // quotient (x + f0 < 512), longer ones have two pieces at most
+  const float inv = 1.0f / (float)n1;
+  auto piece = [&](int x) { return n1 > 256 ? (int)(x + f0 >= n1) : (int)((x + f0 + 0.5f) * inv); };
+  const int x = (tid >> 6) * 63 + lane;  // this lane's face of the run
+  const int q = piece(x), f = x + f0 - q * n1;
+  const bool ok = x <= last;
+  const int i = g.h + f, j = g.h + j0 + p0 + q;
+  const int pos = x + (SW - 1) * q + HW;  // this lane's cell in the LDS row
+  const bool own = ok && lane < 63 && f < g.ix;  // the cell this lane completes
+  // halo cell tid: cell he of piece hq, left (e < HW) or right of it
+  const int hq = tid / (SW - 1), e = tid % (SW - 1);
+  const bool halo = hq <= piece(last);
+  const int l0 = hq == 0 ? 0 : hq * n1 - f0, l1 = min(last, (hq + 1) * n1 - 1 - f0);  // the piece's lanes
+  const int hx = e < HW ? l0 - HW + e : l1 + 1 + e - HW;  // as a lane
+  const int hat = hx + (SW - 1) * hq + HW;
+  const int hi = g.h + hx + f0 - hq * n1, hj = g.h + j0 + p0 + hq;
+  const bool hsens = SENS && halo && e == HW - 1;  // left of the piece's first face
+
+  auto part = [&](const CellAt& m, const RC& r) {
+    constexpr int H = vcross<VO>() / 2;  // r.x[.][H-1], r.x[.][H]: the -1 and +1 neighbours
+    R uym, uyp, vym, vyp, uzm, uzp, wzm, wzp;
+    if constexpr (VISC) {  // DIR 0 cross stencils: u,v along y; u,w along z
+      uym = R(r.x[0][H - 1]); uyp = R(r.x[0][H]);
+      vym = R(r.x[1][H - 1]); vyp = R(r.x[1][H]);
+      uzm = R(r.x[2][H - 1]); uzp = R(r.x[2][H]);
+      wzm = R(r.x[3][H - 1]); wzp = R(r.x[3][H]);
+    } else {
+      uym = R(at(P.u, m, -sy)); uyp = R(at(P.u, m, sy));
+      vym = R(at(P.v, m, -sy)); vyp = R(at(P.v, m, sy));
+      uzm = R(at(P.u, m, -sz)); uzp = R(at(P.u, m, sz));
+      wzm = R(at(P.w, m, -sz)); wzp = R(at(P.w, m, sz));
     }
+    return ducros_yz<R>(g, uym, uyp, vym, vyp, R(at(P.w, m, -sy)), R(at(P.w, m, sy)), uzm, uzp, R(at(P.v, m, -sz)),
+                        R(at(P.v, m, sz)), wzm, wzp);
+  };
+  auto put = [&](int x, const CD& d) {
+    tile[0][x] = d.rho; tile[1][x] = d.u; tile[2][x] = d.v; tile[3][x] = d.w; tile[4][x] = d.p;
+    if constexpr (kUsesT<SCHEME> || VISC) tile[XF::T][x] = d.T;
+    if constexpr (VISC) {
+      tile[XF::mu][x] = d.mu;
+      tile[XF::d][x] = d.d1; tile[XF::d + 1][x] = d.d2; tile[XF::d + 2][x] = d.d3; tile[XF::d + 3][x] = d.d4;
+      if constexpr (VISC == 2) { tile[XF::mt][x] = d.mt; tile[XF::H][x] = d.H; }
+    }
+  };
+  DucrosPart<R> dp{}, hdp{};
+  // cells from the start of the run's first row
+  const int row0 = cidx(g, 0, g.h + j0 + p0, k);
+  const CellAt m{row0, (unsigned)(i + q * sy) * (unsigned)sizeof(S)};
+  const CellAt hm{row0, (unsigned)(hi + hq * sy) * (unsigned)sizeof(S)};
+  RC r, hr;
+  auto take = [&](const CellAt& m, RC& r) { fetch_cell<S, 0, ORDER, SCHEME, VISC, VO, false>(P, g, m, m, r); };
+  auto fill = [&](int x, const RC& r) {
     CD d;
     finish_cell<R, S, 0, ORDER, SCHEME, VISC, VO, false>(g, c, r, d);
-    tile[0][ty][m] = d.rho; tile[1][ty][m] = d.u; tile[2][ty][m] = d.v; tile[3][ty][m] = d.w;
-    tile[4][ty][m] = d.p;
-    if constexpr (kUsesT<SCHEME> || VISC) tile[5][ty][m] = d.T;
-    if constexpr (VISC) {
-      tile[6][ty][m] = d.mu;
-      tile[8][ty][m] = d.d1; tile[9][ty][m] = d.d2; tile[10][ty][m] = d.d3; tile[11][ty][m] = d.d4;
-      if constexpr (VISC == 2) { tile[NF - 2][ty][m] = d.mt; tile[NF - 1][ty][m] = d.H; }
+    put(x, d);
+  };
+  if constexpr (EARLY) {
+    if (halo) take(hm, hr);
+  }
+  if (ok) {
+    take(m, r);
+    if constexpr (SPLIT_SENS) dp = part(m, r);
+    fill(pos, r);
+  }
+  if (halo) {
+    if constexpr (!EARLY) take(hm, hr);
+    if constexpr (SPLIT_SENS) {
+      if (hsens) hdp = part(hm, hr);
     }
+    fill(hat, hr);
   }
   __syncthreads();
   if constexpr (SENS) {
-    if constexpr (SPLIT_SENS) {
-      if (rowok && spos) {
-        const R fd = ducros_x<R>(g, dp, tile[1][ty][m - 1], tile[1][ty][m + 1], tile[2][ty][m - 1],
-                                 tile[2][ty][m + 1], tile[3][ty][m - 1], tile[3][ty][m + 1]);
-        tile[7][ty][m] = fd;
-        if (i >= i0 && i < i0 + XT && i < g.h + g.ix) G(P.s)[cidx(g, i, j, k)] = (S)fd;  // one tile stores a cell
+    auto sensor = [&](int x, int ci, int cj, const DucrosPart<R>& part_yz) {
+      if constexpr (SPLIT_SENS) {
+        return ducros_x<R>(g, part_yz, tile[1][x - 1], tile[1][x + 1], tile[2][x - 1], tile[2][x + 1], tile[3][x - 1],
+                           tile[3][x + 1]);
+      } else {
+        const int n = cidx(g, min(max(ci, 1), g.nx - 2), cj, k);
+        return ducros<R>(g, R(G(P.u)[n - 1]), R(G(P.u)[n + 1]), R(G(P.v)[n - 1]), R(G(P.v)[n + 1]), R(G(P.w)[n - 1]),
+                         R(G(P.w)[n + 1]), R(G(P.u)[n - sy]), R(G(P.u)[n + sy]), R(G(P.v)[n - sy]), R(G(P.v)[n + sy]),
+                         R(G(P.w)[n - sy]), R(G(P.w)[n + sy]), R(G(P.u)[n - sz]), R(G(P.u)[n + sz]), R(G(P.v)[n - sz]),
+                         R(G(P.v)[n + sz]), R(G(P.w)[n - sz]), R(G(P.w)[n + sz]));
       }
-    } else {
-      if (rowok && m >= St::HW - 1 && m <= St::HW + XT && i <= g.nx - 1) {
-        const int ic = min(max(i, 1), g.nx - 2);
-        const int q = cidx(g, ic, j, k);
-        const R fd = ducros<R>(g, R(G(P.u)[q - 1]), R(G(P.u)[q + 1]), R(G(P.v)[q - 1]), R(G(P.v)[q + 1]), R(G(P.w)[q - 1]),
-                               R(G(P.w)[q + 1]), R(G(P.u)[q - sy]), R(G(P.u)[q + sy]), R(G(P.v)[q - sy]), R(G(P.v)[q + sy]),
-                               R(G(P.w)[q - sy]), R(G(P.w)[q + sy]), R(G(P.u)[q - sz]), R(G(P.u)[q + sz]), R(G(P.v)[q - sz]),
-                               R(G(P.v)[q + sz]), R(G(P.w)[q - sz]), R(G(P.w)[q + sz]));
-        tile[7][ty][m] = fd;
-        if (i >= i0 && i < i0 + XT && i < g.h + g.ix) G(P.s)[q] = (S)fd;
-      }
+    };
+    if (ok) {
+      const R fd = sensor(pos, i, j, dp);
+      tile[XF::s][pos] = fd;
+      if (own) G(P.s)[cidx(g, i, j, k)] = (S)fd;  // one run stores a cell
     }
+    if (hsens) tile[XF::s][hat] = sensor(hat, hi, hj, hdp);
     __syncthreads();
   }
-  if (!rowok) return;
-  // face f = i0 - 1 + tx: window cells f-HW+1 .. f+HW = tile positions
-  // tx .. tx+SW-1 (< W for the XT+1 faces the tile's cells need)
+  // face f: window cells f - HW .. f + HW - 1
   R F[5] = {R(0), R(0), R(0), R(0), R(0)};
-  const int f = i0 - 1 + tx;
-  const bool face_ok = tx <= XT && f <= g.h + g.ix - 1;
-  if (face_ok) {
+  if (ok) {
+    const int w0 = pos - HW;
     // The convective and the viscous halves each read their window from the
     // LDS row just before use, which keeps the two halves' inputs out of
     // registers at the same time.
     {
-      CD win[St::SW];
+      CD win[SW];
 #pragma unroll
-      for (int n = 0; n < St::SW; ++n) {
-        win[n].rho = tile[0][ty][tx + n]; win[n].u = tile[1][ty][tx + n]; win[n].v = tile[2][ty][tx + n];
-        win[n].w = tile[3][ty][tx + n]; win[n].p = tile[4][ty][tx + n];
-        if constexpr (kUsesT<SCHEME>) win[n].T = tile[5][ty][tx + n];
+      for (int n = 0; n < SW; ++n) {
+        win[n].rho = tile[0][w0 + n]; win[n].u = tile[1][w0 + n]; win[n].v = tile[2][w0 + n];
+        win[n].w = tile[3][w0 + n]; win[n].p = tile[4][w0 + n];
+        if constexpr (kUsesT<SCHEME>) win[n].T = tile[XF::T][w0 + n];
         if constexpr (SENS) {
-          if (n == St::HW - 1 || n == St::HW) win[n].s = tile[7][ty][tx + n];
+          if (n == HW - 1 || n == HW) win[n].s = tile[XF::s][w0 + n];
         }
       }
-      face_conv<R, 0, ORDER, SCHEME, VISC, VO>(c, tvd, variant, win, F);
+      face_conv<R, 0, ORDER, SCHEME, VISC, VO>(c, a.tvd, a.variant, win, F);
     }
     if constexpr (VISC) {
       OX_SPLIT_FENCE();
-      CD win[St::SW];
+      CD win[SW];
 #pragma unroll
-      for (int n = 0; n < St::SW; ++n) {
-        win[n].u = tile[1][ty][tx + n]; win[n].v = tile[2][ty][tx + n]; win[n].w = tile[3][ty][tx + n];
-        win[n].T = tile[5][ty][tx + n];
-        win[n].mu = tile[6][ty][tx + n];
-        win[n].d1 = tile[8][ty][tx + n]; win[n].d2 = tile[9][ty][tx + n];
-        win[n].d3 = tile[10][ty][tx + n]; win[n].d4 = tile[11][ty][tx + n];
-        if constexpr (VISC == 2) { win[n].mt = tile[NF - 2][ty][tx + n]; win[n].H = tile[NF - 1][ty][tx + n]; }
+      for (int n = 0; n < SW; ++n) {
+        win[n].u = tile[1][w0 + n]; win[n].v = tile[2][w0 + n]; win[n].w = tile[3][w0 + n];
+        win[n].T = tile[XF::T][w0 + n];
+        win[n].mu = tile[XF::mu][w0 + n];
+        win[n].d1 = tile[XF::d][w0 + n]; win[n].d2 = tile[XF::d + 1][w0 + n];
+        win[n].d3 = tile[XF::d + 2][w0 + n]; win[n].d4 = tile[XF::d + 3][w0 + n];
+        if constexpr (VISC == 2) { win[n].mt = tile[XF::mt][w0 + n]; win[n].H = tile[XF::H][w0 + n]; }
       }
       face_visc<R, 0, ORDER, SCHEME, VISC, VO>(c, R(g.inv_dx), win, F);
     }
   }
+  // the right face is the next lane's
   double Fr[5];
 #pragma unroll
   for (int l = 0; l < 5; ++l) Fr[l] = __shfl_down((double)F[l], 1, 64);
-  const int ic = i0 + tx;
-  if (tx < XT && ic < g.h + g.ix) {
+  if (own) {
+    const double cx = a.cd;
 #pragma unroll
-    for (int l = 0; l < 5; ++l) G(Racc)[qidx(g, ic, l, j, k)] = (S)(cx * (-(double)F[l] + Fr[l]));
+    for (int l = 0; l < 5; ++l) G(a.Racc)[qidx(g, i, l, j, k)] = (S)(cx * (-(double)F[l] + Fr[l]));
   }
 }
 
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 __global__ __launch_bounds__(256) void k_sweep_x(SweepArgs<R, S> a) {
-  __shared__ R tile[xsweep_nf<VISC>()][XROWS][64];
-  int bx, by, bz;
-  launch_tile_xzy(bx, by, bz);
-  sweep_x_tile<R, S, ORDER, SCHEME, VISC, VO>(a, bx, by, bz, tile);
+  __shared__ XRunTile<R, ORDER, SCHEME, VISC, VO> lds;
+  sweep_x_run<R, S, ORDER, SCHEME, VISC, VO>(a, xcd_tile(blockIdx.x, gridDim.x), lds);
 }
 
 // ---------------------------------------------------------------------------
 // x sweep over whole rows of a periodic grid whose interior width ix is 64,
-// 128 or 256.  A row tile above spends SW - 1 of its 64 lanes on halo cells,
-// so a row of 256 cells at SW = 6 takes five waves, the fifth with 24 cells.
-// Here a workgroup of 256 lanes holds 256 / ix whole rows, one lane per cell
+// 128 or 256.  The runs above load a second cell in the lanes of a halo and one
+// face in 64 twice; here a workgroup of 256 lanes holds 256 / ix whole rows, one lane per cell
 // and one face per lane (its cell's left face), and the halo positions of the
 // LDS row hold the periodic images of the row's other end.  The face left of
 // the first cell is then the face right of the last: its window cells are the
-// periodic images of that face's window cells.  The row tile computes the
-// same face from the ghost cells, which hold exact copies of those images
-// once a z-sweep epilogue has written the primitive set, so both tiles give
-// the same bits.  Used for such primitive sets only (k_prim takes the ghost
+// periodic images of that face's window cells.  The run computes the same face from the ghost cells, which hold exact copies of those images
+// once a z-sweep epilogue has written the primitive set, so both give the
+// same bits.  Used for such primitive sets only (k_prim takes the ghost
 // layers of an uploaded state as they are), on fully periodic grids, without
 // LES (the ghost SGS fields are copies of the layer next to
 // the boundary), and not for ORDER 2 with the
@@ -864,11 +941,11 @@ __global__ __launch_bounds__(256) void k_sweep_xrow(SweepArgs<R, S> a) {
   using CD = CellData<R, 0, ORDER, SCHEME, VISC, VO>;
   using RC = RawCell<S, VISC, VO>;
   constexpr bool SENS = kUsesSensor<SCHEME, ORDER>;
-  constexpr int NF = xsweep_nf<VISC>();
+  using XF = XFields<ORDER, SCHEME, VISC>;
   constexpr int HW = St::HW, SW = St::SW;
   static_assert(kXRowSweep<ORDER, SCHEME, VISC>, "row sweep for image-ghost schemes only");
   // rows of L + SW - 1 positions: 4 * (63 + SW) covers L = 64 (four rows) to 256 (one)
-  __shared__ R tile[NF][4 * (63 + SW)];
+  __shared__ R tile[XF::N][4 * (63 + SW)];
   __shared__ double edge[4][5];  // each wave's lane-0 face flux
   const Prim<S>& P = a.P;
   const Geom& g = a.g;
@@ -887,7 +964,15 @@ __global__ __launch_bounds__(256) void k_sweep_xrow(SweepArgs<R, S> a) {
   DucrosPart<R> dp{};
   if (rowok) {
     RC rc;
-    fetch_cell<S, 0, ORDER, SCHEME, VISC, VO, false>(P, g, q, 0, rc);
+    // Scalar addresses where the registers that they cost lower no occupancy: FP64
+    // KEEP4 NS 256^3 421 -> 391 us, 128^3 60.6 -> 56.1; SLAU6 NS 128^3 99 -> 108.
+    const auto qa = [&] {
+      if constexpr (SCHEME == KEEP && VISC && sizeof(R) == 8)
+        return CellAt{cidx(g, 0, j - r, k), (unsigned)(i + r * g.nx) * (unsigned)sizeof(S)};
+      else
+        return q;
+    }();
+    fetch_cell<S, 0, ORDER, SCHEME, VISC, VO, false>(P, g, qa, qa, rc);
     if constexpr (SENS) {
       const int sy = g.nx, sz = g.nx * g.ny;
       constexpr int H = vcross<VO>() / 2;
@@ -898,23 +983,23 @@ __global__ __launch_bounds__(256) void k_sweep_xrow(SweepArgs<R, S> a) {
         uzm = R(rc.x[2][H - 1]); uzp = R(rc.x[2][H]);
         wzm = R(rc.x[3][H - 1]); wzp = R(rc.x[3][H]);
       } else {
-        uym = R(G(P.u)[q - sy]); uyp = R(G(P.u)[q + sy]);
-        vym = R(G(P.v)[q - sy]); vyp = R(G(P.v)[q + sy]);
-        uzm = R(G(P.u)[q - sz]); uzp = R(G(P.u)[q + sz]);
-        wzm = R(G(P.w)[q - sz]); wzp = R(G(P.w)[q + sz]);
+        uym = R(at(P.u, qa, -sy)); uyp = R(at(P.u, qa, sy));
+        vym = R(at(P.v, qa, -sy)); vyp = R(at(P.v, qa, sy));
+        uzm = R(at(P.u, qa, -sz)); uzp = R(at(P.u, qa, sz));
+        wzm = R(at(P.w, qa, -sz)); wzp = R(at(P.w, qa, sz));
       }
-      dp = ducros_yz<R>(g, uym, uyp, vym, vyp, R(G(P.w)[q - sy]), R(G(P.w)[q + sy]), uzm, uzp, R(G(P.v)[q - sz]),
-                        R(G(P.v)[q + sz]), wzm, wzp);
+      dp = ducros_yz<R>(g, uym, uyp, vym, vyp, R(at(P.w, qa, -sy)), R(at(P.w, qa, sy)), uzm, uzp, R(at(P.v, qa, -sz)),
+                        R(at(P.v, qa, sz)), wzm, wzp);
     }
     CD d;
     finish_cell<R, S, 0, ORDER, SCHEME, VISC, VO, false>(g, c, rc, d);
-    auto put = [&](int at) {
-      at += rb;
-      tile[0][at] = d.rho; tile[1][at] = d.u; tile[2][at] = d.v; tile[3][at] = d.w; tile[4][at] = d.p;
-      if constexpr (kUsesT<SCHEME> || VISC) tile[5][at] = d.T;
+    auto put = [&](int x) {
+      x += rb;
+      tile[0][x] = d.rho; tile[1][x] = d.u; tile[2][x] = d.v; tile[3][x] = d.w; tile[4][x] = d.p;
+      if constexpr (kUsesT<SCHEME> || VISC) tile[XF::T][x] = d.T;
       if constexpr (VISC) {
-        tile[6][at] = d.mu;
-        tile[8][at] = d.d1; tile[9][at] = d.d2; tile[10][at] = d.d3; tile[11][at] = d.d4;
+        tile[XF::mu][x] = d.mu;
+        tile[XF::d][x] = d.d1; tile[XF::d + 1][x] = d.d2; tile[XF::d + 2][x] = d.d3; tile[XF::d + 3][x] = d.d4;
       }
     };
     put(m);
@@ -924,11 +1009,11 @@ __global__ __launch_bounds__(256) void k_sweep_xrow(SweepArgs<R, S> a) {
   __syncthreads();
   if constexpr (SENS) {
     if (rowok) {
-      const int at = rb + m;
-      const R fd = ducros_x<R>(g, dp, tile[1][at - 1], tile[1][at + 1], tile[2][at - 1], tile[2][at + 1],
-                               tile[3][at - 1], tile[3][at + 1]);
-      tile[7][at] = fd;
-      if (p == L - 1) tile[7][rb + HW - 1] = fd;  // the image left of the row
+      const int x = rb + m;
+      const R fd = ducros_x<R>(g, dp, tile[1][x - 1], tile[1][x + 1], tile[2][x - 1], tile[2][x + 1],
+                               tile[3][x - 1], tile[3][x + 1]);
+      tile[XF::s][x] = fd;
+      if (p == L - 1) tile[XF::s][rb + HW - 1] = fd;  // the image left of the row
       G(P.s)[q] = (S)fd;
     }
     __syncthreads();
@@ -942,9 +1027,9 @@ __global__ __launch_bounds__(256) void k_sweep_xrow(SweepArgs<R, S> a) {
       for (int n = 0; n < SW; ++n) {
         win[n].rho = tile[0][w0 + n]; win[n].u = tile[1][w0 + n]; win[n].v = tile[2][w0 + n];
         win[n].w = tile[3][w0 + n]; win[n].p = tile[4][w0 + n];
-        if constexpr (kUsesT<SCHEME>) win[n].T = tile[5][w0 + n];
+        if constexpr (kUsesT<SCHEME>) win[n].T = tile[XF::T][w0 + n];
         if constexpr (SENS) {
-          if (n == HW - 1 || n == HW) win[n].s = tile[7][w0 + n];
+          if (n == HW - 1 || n == HW) win[n].s = tile[XF::s][w0 + n];
         }
       }
       face_conv<R, 0, ORDER, SCHEME, VISC, VO>(c, a.tvd, a.variant, win, F);
@@ -955,10 +1040,10 @@ __global__ __launch_bounds__(256) void k_sweep_xrow(SweepArgs<R, S> a) {
 #pragma unroll
       for (int n = 0; n < SW; ++n) {
         win[n].u = tile[1][w0 + n]; win[n].v = tile[2][w0 + n]; win[n].w = tile[3][w0 + n];
-        win[n].T = tile[5][w0 + n];
-        win[n].mu = tile[6][w0 + n];
-        win[n].d1 = tile[8][w0 + n]; win[n].d2 = tile[9][w0 + n];
-        win[n].d3 = tile[10][w0 + n]; win[n].d4 = tile[11][w0 + n];
+        win[n].T = tile[XF::T][w0 + n];
+        win[n].mu = tile[XF::mu][w0 + n];
+        win[n].d1 = tile[XF::d][w0 + n]; win[n].d2 = tile[XF::d + 1][w0 + n];
+        win[n].d3 = tile[XF::d + 2][w0 + n]; win[n].d4 = tile[XF::d + 3][w0 + n];
       }
       face_visc<R, 0, ORDER, SCHEME, VISC, VO>(c, R(g.inv_dx), win, F);
     }
@@ -988,25 +1073,16 @@ __global__ __launch_bounds__(256) void k_sweep_xrow(SweepArgs<R, S> a) {
   }
 }
 
-// Persistent batched x sweep: block b handles global tiles b, b + gridDim.x, ...
+// Batched x sweep over the runs of several cases, one workgroup per run: the
+// hardware gives a free slot the next run.  (1024 workgroups that each took every
+// 1024th run left the compute units at half their waves: 156 -> 150 ms for six
+// FP32 requests of 64^3 to 160^3, 60 steps.)
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 __global__ __launch_bounds__(256) void k_sweep_x_batch(const SweepArgs<R, S>* __restrict__ cases,
                                                        const TileMap* __restrict__ map, int ncase, int ntiles) {
-  __shared__ R tile[xsweep_nf<VISC>()][XROWS][64];
-  for (int t = xcd_tile(blockIdx.x, gridDim.x); t < ntiles; t += gridDim.x) {
-    const int ci = find_case(map, ncase, t);
-    const int local = t - map[ci].start, nbx = map[ci].nbx;
-#if OX_XSWEEP_ZMAJOR
-    const int nbz = map[ci].nbz;
-    sweep_x_tile<R, S, ORDER, SCHEME, VISC, VO>(cases[ci], local % nbx, local / (nbx * nbz), (local / nbx) % nbz,
-                                                tile);
-#else
-    const int nby = map[ci].nby;
-    sweep_x_tile<R, S, ORDER, SCHEME, VISC, VO>(cases[ci], local % nbx, (local / nbx) % nby, local / (nbx * nby),
-                                                tile);
-#endif
-    __syncthreads();  // the next tile overwrites the LDS rows
-  }
+  __shared__ XRunTile<R, ORDER, SCHEME, VISC, VO> lds;
+  const int t = xcd_tile(blockIdx.x, ntiles), ci = find_case(map, ncase, t);
+  sweep_x_run<R, S, ORDER, SCHEME, VISC, VO>(cases[ci], t - map[ci].start, lds);
 }
 
 // The residual of one cell and, for the z sweep, the state values its RK

@@ -24,9 +24,7 @@ template <class S> Prim<S> prim_set(const Core& C, int set) {
 
 // Launch grids of the three sweeps of one case (tiles along the three
 // launch dimensions).
-template <int ORDER, int VISC, int VO> dim3 grid_x(const Geom& g) {
-  return dim3(cdiv(g.ix, xtile<ORDER, VISC, VO>()), cdiv(g.iy, XROWS), g.iz);
-}
+inline dim3 grid_x(const Geom& g) { return dim3((unsigned)xrun_blocks(g)); }
 // k_sweep_xrow: 256 / ix rows per workgroup, bands of XROW_BAND rows per plane
 inline dim3 grid_xrow(const Geom& g) {
   return dim3((unsigned)(cdiv(g.iy, XROW_BAND) * g.iz * (XROW_BAND / (256 / g.ix))));
@@ -76,6 +74,7 @@ void make_sweep_args(const Core& C, const StageArgs& sa, double cx, double cy, d
   a3[0] = a;
   a3[0].cd = cx;
   a3[0].lseg = 0;
+  xrun_shape(C.g, a3[0].xrows, a3[0].xwgs);
   a3[1] = a;
   a3[1].cd = cy;
   a3[1].lseg = C.lseg[0];
@@ -87,7 +86,6 @@ void make_sweep_args(const Core& C, const StageArgs& sa, double cx, double cy, d
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 void run_stage(Core& C, const double* Qsrc, const StageArgs& sa, double cx, double cy, double cz) {
   const Geom& g = C.g;
-  const dim3 blk(64, 4, 1);
   prepare_stage<R, S, ORDER, SCHEME, VISC, VO>(C, Qsrc);
   SweepArgs<R, S> a[3];
   make_sweep_args<R, S>(C, sa, cx, cy, cz, a);
@@ -96,7 +94,7 @@ void run_stage(Core& C, const double* Qsrc, const StageArgs& sa, double cx, doub
     rows = xrow_width(g.ix) && !any_bc(g) && C.prim_images[C.cur];
     if (rows) k_sweep_xrow<R, S, ORDER, SCHEME, VISC, VO><<<grid_xrow(g), 256, 0, C.stream>>>(a[0]);
   }
-  if (!rows) k_sweep_x<R, S, ORDER, SCHEME, VISC, VO><<<grid_x<ORDER, VISC, VO>(g), blk, 0, C.stream>>>(a[0]);
+  if (!rows) k_sweep_x<R, S, ORDER, SCHEME, VISC, VO><<<grid_x(g), 256, 0, C.stream>>>(a[0]);
   prof_mark(C, "sweep_x");
   k_sweep_line<R, S, ORDER, SCHEME, VISC, VO, 1, EP_RHS><<<grid_y(g, a[1].lseg), line_block(), 0, C.stream>>>(a[1]);
   prof_mark(C, "sweep_y");
@@ -125,13 +123,12 @@ void run_stage(Core& C, const double* Qsrc, const StageArgs& sa, double cx, doub
 // viscosity first, as in prepare_stage).
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 void run_stage_batch(const BatchGroupLaunch& L) {
-  const dim3 blk(64, 4, 1);
   using A = SweepArgs<R, S>;
   if constexpr (VISC == 2) {
     k_les_mut_batch<R, S><<<L.grid_les, 256, 0, L.stream>>>((const A*)L.args[0], L.map_les, L.ncase, L.ntiles_les);
   }
   k_sweep_x_batch<R, S, ORDER, SCHEME, VISC, VO>
-      <<<L.grid[0], blk, 0, L.stream>>>((const A*)L.args[0], L.map[0], L.ncase, L.ntiles[0]);
+      <<<L.grid[0], 256, 0, L.stream>>>((const A*)L.args[0], L.map[0], L.ncase, L.ntiles[0]);
   k_sweep_line_batch<R, S, ORDER, SCHEME, VISC, VO, 1, EP_RHS>
       <<<L.grid[1], line_block(), 0, L.stream>>>((const A*)L.args[1], L.map[1], L.ncase, L.ntiles[1]);
 #define OX_ZB(E)                                         \
@@ -180,7 +177,6 @@ template <class R, class S, int ORDER, int SCHEME, int VISC, int VO> int line_oc
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO> BatchOps batch_ops() {
   BatchOps o;
   o.args_bytes = sizeof(SweepArgs<R, S>);
-  o.xt = xtile<ORDER, VISC, VO>();
   o.prepare = &prepare_stage<R, S, ORDER, SCHEME, VISC, VO>;
   o.make_args = &make_sweep_args_erased<R, S>;
   o.launch = &run_stage_batch<R, S, ORDER, SCHEME, VISC, VO>;
