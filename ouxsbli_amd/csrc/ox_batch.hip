@@ -3,7 +3,7 @@
 //
 // Every admitted case is an ox_solver whose kernels run on the engine's
 // stream.  Cases with the same kernel specialisation, precision and RK scheme
-// form a group; one RK stage of a group is three persistent launches (x, y, z
+// form a group; one RK stage of a group is three launches (x, y, z
 // sweeps; one fused launch for 2-D groups) over the concatenated tiles of its
 // cases, each case's tiles reading that case's descriptor.  A 3-D case's
 // descriptors depend on its primitive-set parity, which flips every stage,
@@ -45,7 +45,6 @@ int ox2d_get_state(ox2d_solver* s, double* Q);
 
 namespace {
 
-constexpr int kMaxGrid = 1024;  // persistent blocks per launch (4 per CU on 256 CUs)
 constexpr size_t kMaxArgs = 2048;
 static_assert(sizeof(ox::SweepArgs<double, double>) <= kMaxArgs, "sweep descriptor size");
 static_assert(sizeof(ox::SweepArgs<float, float>) <= kMaxArgs, "sweep descriptor size");
@@ -150,7 +149,7 @@ int ensure_device(char** p, size_t* cap, size_t need) {
 }
 
 // Groups and the per-step launch plan for the current active cases: tile
-// maps (uploaded here), descriptor offsets, persistent grid sizes.  The
+// maps (uploaded here), descriptor offsets, launch sizes.  The
 // descriptors of 2-D groups do not change from step to step and are written
 // here; those of 3-D groups are refreshed before every step.
 int build_plan(ox_batch* b) {
@@ -286,13 +285,12 @@ int build_plan(ox_batch* b) {
         for (int d = 0; d < 3; ++d) {
           L.map[d] = b->d_map + map_off[gi] + (size_t)d * n;
           L.ntiles[d] = ntiles[gi][d];
-          // the x sweep takes one workgroup per run
-          L.grid[d] = d == 0 ? ntiles[gi][0] : std::max(1, std::min(ntiles[gi][d], kMaxGrid));
+          L.grid[d] = ntiles[gi][d];
         }
         if (G.les) {
           L.map_les = b->d_map + map_off[gi] + (size_t)3 * n;
           L.ntiles_les = ntiles_les[gi];
-          L.grid_les = std::max(1, std::min(ntiles_les[gi], kMaxGrid));
+          L.grid_les = ntiles_les[gi];
         }
       } else {
         L.ntiles[0] = ntiles[gi][0];

@@ -70,7 +70,7 @@ inline void finish_stage(Core& C, const StageArgs& sa) {
 
 // ---------------------------------------------------------------------------
 // Batched stages.  The cases of one group share a kernel specialisation; one
-// stage of the whole group is three persistent launches (x, y, z sweeps)
+// stage of the whole group is three launches (x, y, z sweeps)
 // over the concatenated tiles of its cases.
 // ---------------------------------------------------------------------------
 struct TileMap;
@@ -81,7 +81,7 @@ struct BatchGroupLaunch {
   const void* args[3];     // device arrays of the per-case sweep descriptors (x, y, z)
   const TileMap* map[3];   // device tile maps (x, y, z)
   int ntiles[3];
-  int grid[3];             // persistent grid sizes
+  int grid[3];             // workgroups: the tiles (2-D: a persistent grid)
   int ep;                  // RK epilogue of the stage
   // LES groups: the SGS viscosity
   const TileMap* map_les;

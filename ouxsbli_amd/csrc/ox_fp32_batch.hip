@@ -1,5 +1,5 @@
-// ox_fp32_batch.hip -- FP32-bulk specialisations of the batched (multi-case,
-// persistent) stage launches.
+// ox_fp32_batch.hip -- FP32-bulk specialisations of the batched (multi-case)
+// stage launches.
 #include "ox_stage_impl.hpp"
 
 namespace ox {

@@ -1,5 +1,5 @@
 // ox_fp64_batch.hip -- FP64 plain-form specialisations of the batched
-// (multi-case, persistent) stage launches.  Same kernels bodies as the
+// (multi-case) stage launches.  Same kernels bodies as the
 // single-case launches; built with -ffp-contract=off like them.
 #include "ox_stage_impl.hpp"
 

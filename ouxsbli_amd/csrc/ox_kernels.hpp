@@ -1073,10 +1073,11 @@ __global__ __launch_bounds__(256) void k_sweep_xrow(SweepArgs<R, S> a) {
   }
 }
 
-// Batched x sweep over the runs of several cases, one workgroup per run: the
-// hardware gives a free slot the next run.  (1024 workgroups that each took every
-// 1024th run left the compute units at half their waves: 156 -> 150 ms for six
-// FP32 requests of 64^3 to 160^3, 60 steps.)
+// Batched sweeps over the tiles of several cases, one workgroup per tile, as in a
+// lone case's launch: the hardware gives a free slot the next tile.  1024
+// workgroups that each walked every 1024th tile left the compute units at half
+// their waves and finished unevenly: six FP32 requests of 64^3 to 160^3, 60 steps,
+// 156 -> 150 ms for the x sweep and 139 with the y and z sweeps.
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 __global__ __launch_bounds__(256) void k_sweep_x_batch(const SweepArgs<R, S>* __restrict__ cases,
                                                        const TileMap* __restrict__ map, int ncase, int ntiles) {
@@ -1428,32 +1429,26 @@ __global__ __launch_bounds__(256, line_waves<VISC>()) void k_sweep_line(SweepArg
   sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(a, t % gx, t / gx, ring);
 }
 
-// Persistent batched y / z sweep over the tiles of several cases.
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO, int DIR, int EP>
 __global__ __launch_bounds__(256, line_waves<VISC>()) void k_sweep_line_batch(
     const SweepArgs<R, S>* __restrict__ cases, const TileMap* __restrict__ map, int ncase, int ntiles) {
   __shared__ R ring[std::max(1, ring_values<R, ORDER, SCHEME, VISC, VO>())];
-  for (int t = xcd_tile(blockIdx.x, gridDim.x); t < ntiles; t += gridDim.x) {
-    const int ci = find_case(map, ncase, t);
-    const int local = t - map[ci].start, nbx = map[ci].nbx;
-    sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(cases[ci], local % nbx, local / nbx, ring);
-  }
+  const int t = xcd_tile(blockIdx.x, ntiles), ci = find_case(map, ncase, t);
+  const int local = t - map[ci].start, nbx = map[ci].nbx;
+  sweep_line_tile<R, S, ORDER, SCHEME, VISC, VO, DIR, EP>(cases[ci], local % nbx, local / nbx, ring);
 }
 
-// Persistent batched SGS viscosity of LES cases over the tiles of several
-// cases, reading each case's x-sweep descriptor: the primitive set the stage
-// reads, the geometry and the constants.
+// Batched SGS viscosity of LES cases over the tiles of several cases, reading
+// each case's x-sweep descriptor: the primitive set the stage reads, the
+// geometry and the constants.
 template <class R, class S>
 __global__ __launch_bounds__(256) void k_les_mut_batch(const SweepArgs<R, S>* __restrict__ cases,
                                                        const TileMap* __restrict__ map, int ncase, int ntiles) {
   __shared__ LesPlanes<R> pl;
-  for (int t = xcd_tile(blockIdx.x, gridDim.x); t < ntiles; t += gridDim.x) {
-    const int ci = find_case(map, ncase, t);
-    const int local = t - map[ci].start, nbx = map[ci].nbx, nby = map[ci].nby;
-    const SweepArgs<R, S>& a = cases[ci];
-    les_mut_tile<S, R>(a.P, a.g, a.c, local % nbx, (local / nbx) % nby, local / (nbx * nby), pl);
-    __syncthreads();  // the next tile overwrites the planes
-  }
+  const int t = xcd_tile(blockIdx.x, ntiles), ci = find_case(map, ncase, t);
+  const int local = t - map[ci].start, nbx = map[ci].nbx, nby = map[ci].nby;
+  const SweepArgs<R, S>& a = cases[ci];
+  les_mut_tile<S, R>(a.P, a.g, a.c, local % nbx, (local / nbx) % nby, local / (nbx * nby), pl);
 }
 
 }  // namespace ox

@@ -119,7 +119,7 @@ void run_stage(Core& C, const double* Qsrc, const StageArgs& sa, double cx, doub
   finish_stage(C, sa);
 }
 
-// One stage of a group of cases: three persistent launches (LES: the SGS
+// One stage of a group of cases: three launches (LES: the SGS
 // viscosity first, as in prepare_stage).
 template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 void run_stage_batch(const BatchGroupLaunch& L) {
