@@ -95,8 +95,7 @@ int solver2d_create(const ox2d_config* cfg, hipStream_t shared, ox2d_solver** ou
     delete s;
     return ox_fail(OX_EUNSUPPORTED, "no 2-D specialisation for this order and scheme");
   }
-  s->g.init(*cfg, ox2::tile_rows_of(cfg->precision));
-  s->ntiles = s->g.nbx * s->g.nby;
+  s->g.init(*cfg);
   auto fail = [&](int code, const char* msg) {
     ox2d_destroy(s);
     return ox_fail(code, msg);
@@ -117,9 +116,7 @@ int solver2d_create(const ox2d_config* cfg, hipStream_t shared, ox2d_solver** ou
   if (hipMemcpyAsync(s->d_args, h.data(), h.size(), hipMemcpyHostToDevice, s->stream) != hipSuccess ||
       hipStreamSynchronize(s->stream) != hipSuccess)
     return fail(OX_EDEVICE, "descriptor upload failed");
-  int cap = s->launch[0].max_blocks();
-  for (int st = 1; st < 3; ++st) cap = std::min(cap, s->launch[st].max_blocks());
-  s->grid = ox2::grid2(s->ntiles, cap);
+  s->rows = ox2::pick_rows(s->launch, s->g.ntiles(0));
   *out = s;
   return OX_OK;
 }
@@ -159,7 +156,8 @@ int ox2d_step(ox2d_solver* s, int32_t nsteps) {
   OX_HIP(hipSetDevice(s->cfg.device));
   OX_HIP(hipEventRecord(s->ev0, s->stream));
   for (int t = 0; t < nsteps; ++t)
-    for (int st = 0; st < 3; ++st) s->launch[st].launch(s->d_args + st * s->args_bytes, 1, s->ntiles, s->grid, s->stream);
+    for (int st = 0; st < 3; ++st)
+      s->launch[st].launch[s->rows](s->d_args + st * s->args_bytes, 1, s->g.ntiles(s->rows), s->stream);
   OX_HIP(hipGetLastError());
   OX_HIP(hipEventRecord(s->ev1, s->stream));
   OX_HIP(hipEventSynchronize(s->ev1));

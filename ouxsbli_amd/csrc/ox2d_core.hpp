@@ -12,12 +12,20 @@
 
 namespace ox2 {
 
-// A stage launcher of one kernel specialisation and the number of its
-// workgroups the device holds at once (the persistent grid's cap).
+// The stage launchers of one kernel specialisation, for tiles of ROWS[0] and of
+// ROWS[1] rows, and the number of its ROWS[0]-row workgroups that the device holds
+// at once.
 struct Launch2 {
-  void (*launch)(const void* args, int ncase, int ntiles, int grid, hipStream_t stream);
-  int (*max_blocks)();
+  void (*launch[2])(const void* args, int ncase, int ntiles, hipStream_t stream);
+  int (*few_tiles)();
 };
+
+// Which of the two a launch of `ntiles` ROWS[0]-row tiles uses.
+inline int pick_rows(const Launch2 l[3], long long ntiles) {
+  for (int st = 0; st < 3; ++st)
+    if (ntiles > l[st].few_tiles()) return 1;
+  return 0;
+}
 
 // Specialisation key of a 2-D case: (ORDER, SCHEME).
 inline int key2(int order, int scheme) { return order * 10 + scheme; }
@@ -34,9 +42,10 @@ struct Geom2 {
   double J, dtdx, dtdy, sx, sy, g1;
   double qin[4], qpost[4];
   ox::HostConsts hc;
-  int nbx, nby;
+  int nbx, nby[2];  // tiles, of either height
+  int ntiles(int rows) const { return nbx * nby[rows]; }
 
-  void init(const ox2d_config& c, int tile_rows) {
+  void init(const ox2d_config& c) {
     ox_config c3{};
     c3.nx = c3.ny = c3.nz = 8;
     c3.order = 2;
@@ -59,7 +68,7 @@ struct Geom2 {
     bc_state(c.inflow, Jt, qin);
     bc_state(c.post, Jt, qpost);
     nbx = (c.nx - 2 + TX - 1) / TX;
-    nby = (c.ny - 2 + tile_rows - 1) / tile_rows;
+    for (int r = 0; r < 2; ++r) nby[r] = (c.ny - 2 + ROWS[r] - 1) / ROWS[r];
   }
   void bc_state(const double* s, double Jt, double* q) const {
     q[0] = s[0] * Jt;
@@ -68,8 +77,6 @@ struct Geom2 {
     q[3] = (s[3] * hc.over_gamma_1 + 0.5 * s[0] * (s[1] * s[1] + s[2] * s[2])) * Jt;
   }
 };
-
-inline int tile_rows_of(int precision) { return precision == OX_PREC_FP64 ? tile_rows<double>() : tile_rows<float>(); }
 
 // RK3 stage st (0-based) on the buffers A (= Q^n), B, C: source, Q^n,
 // output and the coefficients of calc_time_dev.f90.fypp:79-93.
@@ -127,14 +134,6 @@ inline void write_args2(const ox2d_config& c, const Geom2& g, double* const buf[
   else *(Args2<float>*)out = make_args2<float>(c, g, buf, st, tile0);
 }
 
-// Persistent grid: the tiles, rounded up to a multiple of 8 (whole XCD
-// rounds), capped at what the device holds at once.
-inline int grid2(int ntiles, int cap) {
-  int g = ntiles > 8 ? (ntiles + 7) / 8 * 8 : ntiles;
-  if (g > cap) g = cap / 8 * 8 > 0 ? cap / 8 * 8 : cap;
-  return g < 1 ? 1 : g;
-}
-
 }  // namespace ox2
 
 // The handle behind ox2d_solver.
@@ -146,7 +145,7 @@ struct ox2d_solver {
   char* d_args = nullptr;                          // the three stage descriptors
   size_t args_bytes = 0;
   ox2::Launch2 launch[3]{};
-  int ntiles = 0, grid = 0;
+  int rows = 0;  // which tiles a launch of this case alone uses
   hipStream_t stream = nullptr, own_stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0.0;

@@ -7,16 +7,17 @@
 
 namespace ox2 {
 
-template <class R, int ORDER, int SCHEME, int EP>
-void launch2(const void* args, int ncase, int ntiles, int grid, hipStream_t stream) {
-  k2d_stage<R, ORDER, SCHEME, EP><<<grid, 256, 0, stream>>>((const Args2<R>*)args, ncase, ntiles);
+template <class R, int ORDER, int SCHEME, int EP, int ROW>
+void launch2(const void* args, int ncase, int ntiles, hipStream_t stream) {
+  k2d_stage<R, ORDER, SCHEME, EP, ROW><<<ntiles, LANES, 0, stream>>>((const Args2<R>*)args, ncase);
 }
 
-template <class R, int ORDER, int SCHEME, int EP> int max_blocks2() {
+template <class R, int ORDER, int SCHEME, int EP> int few_tiles() {
   static int cap = 0;
   if (cap == 0) {
     int occ = 0, dev = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k2d_stage<R, ORDER, SCHEME, EP>, 256, 0) != hipSuccess)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k2d_stage<R, ORDER, SCHEME, EP, ROWS[0]>, LANES, 0) !=
+        hipSuccess)
       occ = 1;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -26,10 +27,14 @@ template <class R, int ORDER, int SCHEME, int EP> int max_blocks2() {
   return cap;
 }
 
+template <class R, int ORDER, int SCHEME, int EP> constexpr Launch2 entry2() {
+  return {{&launch2<R, ORDER, SCHEME, EP, ROWS[0]>, &launch2<R, ORDER, SCHEME, EP, ROWS[1]>},
+          &few_tiles<R, ORDER, SCHEME, EP>};
+}
 template <class R, int ORDER, int SCHEME> void table2(Launch2 out[3]) {
-  out[0] = {&launch2<R, ORDER, SCHEME, EP2_S1>, &max_blocks2<R, ORDER, SCHEME, EP2_S1>};
-  out[1] = {&launch2<R, ORDER, SCHEME, EP2_S2>, &max_blocks2<R, ORDER, SCHEME, EP2_S2>};
-  out[2] = {&launch2<R, ORDER, SCHEME, EP2_S3>, &max_blocks2<R, ORDER, SCHEME, EP2_S3>};
+  out[0] = entry2<R, ORDER, SCHEME, EP2_S1>();
+  out[1] = entry2<R, ORDER, SCHEME, EP2_S2>();
+  out[2] = entry2<R, ORDER, SCHEME, EP2_S3>();
 }
 
 // Supported (ORDER, SCHEME) pairs of the 2-D path.

@@ -15,11 +15,10 @@
 //      arithmetic type R;
 //   2. the Ducros sensor on the cross-shaped set of points the tile's faces
 //      read (boundary points take their inner neighbour's value);
-//   3. the x faces and y faces of the tile into LDS, each with the order its
-//      distance to the boundary allows (6-, 4- or 2-point);
-//   4. per cell: R = cx dE + cy dF in FP64 (the x part as soon as the x
-//      faces are done, kept in registers while the y faces reuse their
-//      LDS), the RK combination in FP64, the new state and -- for cells next
+//   3. the x faces and y faces of the tile into LDS, by one half of the lanes
+//      each, with the order a face's distance to the boundary allows (6-, 4-
+//      or 2-point);
+//   4. per cell: R = cx dE + cy dF in FP64, the RK combination in FP64, the new state and -- for cells next
 //      to the boundary -- the boundary points of the oblique-shock
 //      conditions, from the new values.
 //
@@ -33,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include "ox_physics.hpp"
+#include "ox_xcd.hpp"
 
 namespace ox2 {
 
@@ -66,34 +66,32 @@ template <class R> struct Args2 {
 };
 
 constexpr int TX = 64;
-// Rows per tile.  11 FP32 rows: 715 x faces, 768 y faces and 704 cells
-// keep the 256 threads busy in three passes each, and 34 KiB of LDS (107
-// VGPRs) lets four workgroups share a CU.  4 FP64 rows: 35 KiB of LDS and
-// 124 VGPRs, also four per CU.
-#ifndef OX2_ROWS_FP64
-#define OX2_ROWS_FP64 4
-#endif
-#ifndef OX2_ROWS_FP32
-#define OX2_ROWS_FP32 11
-#endif
-template <class R> constexpr int tile_rows() { return sizeof(R) == 8 ? OX2_ROWS_FP64 : OX2_ROWS_FP32; }
+// Rows per tile TY: 3 where all tiles of a launch are in flight at once, 7
+// otherwise.  A workgroup has 512 lanes, four waves for the x faces and four for
+// the y faces at the same time.  With 3 rows each wave has one face per lane (195 and
+// 256 faces), so a stage is one face computation deep: in a launch that leaves
+// the chip's slots half empty nothing else hides that chain.  7 rows are two
+// faces per lane with few idle lanes (455 and 512 of 512), and a halo of 13 / 7
+// instead of 9 / 3.  Time of a stage (us), 256 lanes that did the x faces, then
+// the y faces, of 4 (FP64) or 11 (FP32) rows -> now: SLAU6 FP64 255 x 127 12.4 ->
+// 7.3, 511 x 255 14.3 -> 11.5, 1023 x 511 33.5 -> 28.8, 2047 x 1023 111 -> 90; FP32 15.2
+// -> 5.1, 15.2 -> 7.1, 19.3 -> 17.1, 54 -> 46.  On either side of the line: 511 x 255, 680
+// tiles of 3 rows, FP64 (512 in flight) 13.8 with 3 rows and 11.5 with 7, FP32
+// (1024) 7.1 and 8.3.  11 and 15 rows were slower (2047 x 1023 FP32 49 and 54).
+constexpr int ROWS[2] = {3, 7};
+constexpr int LANES = 512;
 // halo of the LDS tile: the stencil half-width, at least 2 where the sensor
 // (2nd-order central differences at the points next to the faces) is needed
 template <int ORDER> constexpr int halo() { return ORDER == 6 ? 3 : (ORDER == 4 ? 2 : 1); }
 
-template <class R, int ORDER> struct Tile2 {
-  static constexpr int TY = tile_rows<R>();
+template <class R, int ORDER, int TY_> struct Tile2 {
+  static constexpr int TY = TY_;
   static constexpr int HL = halo<ORDER>();
   static constexpr int W = TX + 2 * HL, H = TY + 2 * HL;
   R prim[4][H][W];               // rho, u, v, p
   R sens[TY + 2][TX + 2];        // Ducros sensor, points x0-1..x0+TX, y0-1..y0+TY
-  // face fluxes: first the x faces x0-1..x0+TX-1 of the tile rows, then --
-  // once each cell holds its x differences in registers -- the y faces
-  // y0-1..y0+TY-1 of the tile columns in the same storage
-  union {
-    R E[4][TY][TX + 1];
-    R F[4][TY + 1][TX];
-  } fl;
+  R E[4][TY][TX + 1];            // x face fluxes x0-1..x0+TX-1 of the tile rows
+  R F[4][TY + 1][TX];            // y face fluxes y0-1..y0+TY-1 of the tile columns
 };
 
 // The Ducros sensor of one interior point from the velocity neighbours
@@ -205,9 +203,9 @@ __device__ __forceinline__ void store_q(double* __restrict__ Q, int nx, int i, i
 
 // One tile: interior cells x0..x0+TX-1, y0..y0+TY-1 (0-based point indices;
 // interior points are 1..nx-2, 1..ny-2).
-template <class R, int ORDER, int SCHEME, int EP>
-__device__ __forceinline__ void stage_tile(const Args2<R>& a, int tx, int ty, Tile2<R, ORDER>& T) {
-  using TL = Tile2<R, ORDER>;
+template <class R, int ORDER, int SCHEME, int EP, int ROW>
+__device__ __forceinline__ void stage_tile(const Args2<R>& a, int tx, int ty, Tile2<R, ORDER, ROW>& T) {
+  using TL = Tile2<R, ORDER, ROW>;
   constexpr int TY = TL::TY, HL = TL::HL, W = TL::W, H = TL::H;
   constexpr int M0 = 3 - ORDER / 2, M1 = 2 + ORDER / 2;  // stencil points f-2+m read, m in [M0, M1]
   const int tid = threadIdx.x;
@@ -217,7 +215,7 @@ __device__ __forceinline__ void stage_tile(const Args2<R>& a, int tx, int ty, Ti
 
   // 1. primitives of the tile and its halo (calc_quantities_2D), recovered in
   //    FP64; points outside the case are zero and never read by a face
-  for (int k = tid; k < W * H; k += 256) {
+  for (int k = tid; k < W * H; k += LANES) {
     const int rx = k % W, ry = k / W;
     const int i = x0 - HL + rx, j = y0 - HL + ry;
     R pr[4] = {R(0), R(0), R(0), R(0)};
@@ -244,7 +242,7 @@ __device__ __forceinline__ void stage_tile(const Args2<R>& a, int tx, int ty, Ti
   //    its inner neighbour (calc_hybrid.f90:39-50)
   const bool sensed = ORDER >= 4 && a.tvd == OX_TVD_HYBRID;
   if (sensed) {
-    for (int k = tid; k < (TX + 2) * (TY + 2); k += 256) {
+    for (int k = tid; k < (TX + 2) * (TY + 2); k += LANES) {
       const int sx = k % (TX + 2), sy = k / (TX + 2);
       if ((sx == 0 || sx == TX + 1) && (sy == 0 || sy == TY + 1)) continue;
       const int i = x0 - 1 + sx, j = y0 - 1 + sy;
@@ -256,74 +254,61 @@ __device__ __forceinline__ void stage_tile(const Args2<R>& a, int tx, int ty, Ti
     __syncthreads();
   }
 
-  // 3a. x faces f = x0-1..xlast (0-based: between points f and f+1) of rows y0..ylast
-  for (int k = tid; k < (TX + 1) * TY; k += 256) {
-    const int fx = k % (TX + 1), fy = k / (TX + 1);
-    const int f = x0 - 1 + fx, j = y0 + fy;
-    if (f > xlast || j > ylast) continue;
-    R st[4][6] = {};
+  // 3. first half of the lanes: x faces f = x0-1..xlast (0-based: between points f and f+1) of rows y0..ylast
+  //    second half: y faces g = y0-1..ylast of columns x0..xlast
+  if (tid < LANES / 2) {
+    for (int k = tid; k < (TX + 1) * TY; k += LANES / 2) {
+      const int fx = k % (TX + 1), fy = k / (TX + 1);
+      const int f = x0 - 1 + fx, j = y0 + fy;
+      if (f > xlast || j > ylast) continue;
+      R st[4][6] = {};
 #pragma unroll
-    for (int m = 0; m < 6; ++m) {
-      if (m < M0 || m > M1) continue;
-      const int lx = f - 2 + m - (x0 - HL);
+      for (int m = 0; m < 6; ++m) {
+        if (m < M0 || m > M1) continue;
+        const int lx = f - 2 + m - (x0 - HL);
 #pragma unroll
-      for (int v = 0; v < 4; ++v) st[v][m] = T.prim[v][fy + HL][lx];
+        for (int v = 0; v < 4; ++v) st[v][m] = T.prim[v][fy + HL][lx];
+      }
+      const R fs = sensed ? R(0.5) * (T.sens[fy + 1][fx] + T.sens[fy + 1][fx + 1]) : R(0);
+      R Fl[4];
+      face2<R, ORDER, SCHEME, 0>(a, f + 1, nx, st, fs, Fl);
+#pragma unroll
+      for (int l = 0; l < 4; ++l) T.E[l][fy][fx] = Fl[l];
     }
-    const R fs = sensed ? R(0.5) * (T.sens[fy + 1][fx] + T.sens[fy + 1][fx + 1]) : R(0);
-    R Fl[4];
-    face2<R, ORDER, SCHEME, 0>(a, f + 1, nx, st, fs, Fl);
+  } else {
+    for (int k = tid - LANES / 2; k < TX * (TY + 1); k += LANES / 2) {
+      const int gx = k % TX, gy = k / TX;
+      const int i = x0 + gx, g = y0 - 1 + gy;
+      if (i > xlast || g > ylast) continue;
+      R st[4][6] = {};
 #pragma unroll
-    for (int l = 0; l < 4; ++l) T.fl.E[l][fy][fx] = Fl[l];
+      for (int m = 0; m < 6; ++m) {
+        if (m < M0 || m > M1) continue;
+        const int ly = g - 2 + m - (y0 - HL);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) st[v][m] = T.prim[v][ly][gx + HL];
+      }
+      const R fs = sensed ? R(0.5) * (T.sens[gy][gx + 1] + T.sens[gy + 1][gx + 1]) : R(0);
+      R Fl[4];
+      face2<R, ORDER, SCHEME, 1>(a, g + 1, ny, st, fs, Fl);
+#pragma unroll
+      for (int l = 0; l < 4; ++l) T.F[l][gy][gx] = Fl[l];
+    }
   }
   __syncthreads();
 
-  // 4a. x part of the residual, R = cx * (-E_i + E_i+1) (calc_R,
-  //     calc_steps.f90:17-21), in registers: cell k = tid + 256 m
-  constexpr int NC = (TX * TY + 255) / 256;
-  double Rc[NC][4];
-#pragma unroll
-  for (int m = 0; m < NC; ++m) {
-    const int k = tid + 256 * m;
-    const int rx = k % TX, ry = k / TX;
-    if (k < TX * TY && x0 + rx <= xlast && y0 + ry <= ylast) {
-#pragma unroll
-      for (int l = 0; l < 4; ++l) Rc[m][l] = a.cx * (-(double)T.fl.E[l][ry][rx] + (double)T.fl.E[l][ry][rx + 1]);
-    }
-  }
-  __syncthreads();
-
-  // 3b. y faces g = y0-1..ylast of columns x0..xlast
-  for (int k = tid; k < TX * (TY + 1); k += 256) {
-    const int gx = k % TX, gy = k / TX;
-    const int i = x0 + gx, g = y0 - 1 + gy;
-    if (i > xlast || g > ylast) continue;
-    R st[4][6] = {};
-#pragma unroll
-    for (int m = 0; m < 6; ++m) {
-      if (m < M0 || m > M1) continue;
-      const int ly = g - 2 + m - (y0 - HL);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) st[v][m] = T.prim[v][ly][gx + HL];
-    }
-    const R fs = sensed ? R(0.5) * (T.sens[gy][gx + 1] + T.sens[gy + 1][gx + 1]) : R(0);
-    R Fl[4];
-    face2<R, ORDER, SCHEME, 1>(a, g + 1, ny, st, fs, Fl);
-#pragma unroll
-    for (int l = 0; l < 4; ++l) T.fl.F[l][gy][gx] = Fl[l];
-  }
-  __syncthreads();
-
-  // 4b. y part of the residual (calc_steps.f90:23-27), RK combination,
-  //     boundary points
-#pragma unroll
-  for (int m = 0; m < NC; ++m) {
-    const int k = tid + 256 * m;
+  // 4. residual, R = cx * (-E_i + E_i+1) + cy * (-F_j + F_j+1) (calc_R,
+  //    calc_steps.f90:17-27), RK combination, boundary points
+  for (int k = tid; k < TX * TY; k += LANES) {
     const int rx = k % TX, ry = k / TX;
     const int i = x0 + rx, j = y0 + ry;
-    if (k >= TX * TY || i > xlast || j > ylast) continue;
+    if (i > xlast || j > ylast) continue;
     double Rr[4];
 #pragma unroll
-    for (int l = 0; l < 4; ++l) Rr[l] = Rc[m][l] + a.cy * (-(double)T.fl.F[l][ry][rx] + (double)T.fl.F[l][ry + 1][rx]);
+    for (int l = 0; l < 4; ++l) {
+      Rr[l] = a.cx * (-(double)T.E[l][ry][rx] + (double)T.E[l][ry][rx + 1]);
+      Rr[l] = Rr[l] + a.cy * (-(double)T.F[l][ry][rx] + (double)T.F[l][ry + 1][rx]);
+    }
     double qs[4], qn[4];
     load_q(a.Qs, nx, ny, i, j, qs);
     if constexpr (EP == EP2_S1) {
@@ -370,23 +355,17 @@ __device__ __forceinline__ int find_case2(const Args2<R>* __restrict__ args, int
   return lo;
 }
 
-// One RK stage over the tiles of `ncase` cases; persistent: each workgroup
-// strides over the tiles.  Workgroups are dealt to the eight XCDs round
-// robin; the logical index groups consecutive tiles (which share halo rows)
-// on one XCD's L2 when the grid is a multiple of 8.
-template <class R, int ORDER, int SCHEME, int EP>
-__global__ __launch_bounds__(256) void k2d_stage(const Args2<R>* __restrict__ args, int ncase, int ntiles) {
-  __shared__ Tile2<R, ORDER> T;
-  const int G = gridDim.x;
-  const int b = blockIdx.x;
-  const int L = (G % 8 == 0) ? (b % 8) * (G / 8) + b / 8 : b;
-  for (int t = L; t < ntiles; t += G) {
-    const int ci = find_case2(args, ncase, t);
-    const Args2<R>& a = args[ci];
-    const int local = t - a.tile0;
-    stage_tile<R, ORDER, SCHEME, EP>(a, local % a.nbx, local / a.nbx, T);
-    __syncthreads();  // the next tile overwrites the LDS
-  }
+// One RK stage over the tiles of `ncase` cases, one workgroup per tile.  (A
+// launch of the workgroups that the device holds at once, each walking every
+// n-th tile, took 52 us for an FP32 stage of 2047 x 1023 where this takes 46, and 51
+// ms for 150 steps of 64 FP32 cases of 257 x 129 where this takes 45.)
+template <class R, int ORDER, int SCHEME, int EP, int ROW>
+__global__ __launch_bounds__(LANES) void k2d_stage(const Args2<R>* __restrict__ args, int ncase) {
+  __shared__ Tile2<R, ORDER, ROW> T;
+  const int t = ox::xcd_tile(blockIdx.x, gridDim.x, true);
+  const Args2<R>& a = args[find_case2(args, ncase, t)];
+  const int local = t - a.tile0;
+  stage_tile<R, ORDER, SCHEME, EP, ROW>(a, local % a.nbx, local / a.nbx, T);
 }
 
 }  // namespace ox2

@@ -76,6 +76,7 @@ struct BGroup {
   bool les;
   ox::BatchOps ops;
   ox2::Launch2 launch2[3];
+  int rows = 0;  // 2-D: which tiles its launches use
   std::vector<BCase*> members;
 };
 
@@ -223,7 +224,10 @@ int build_plan(ox_batch* b) {
     std::array<int, 3> nt{0, 0, 0};
     int nl = 0;
     if (G.dim == 2) {
-      for (BCase* c : G.members) nt[0] += c->s2->ntiles;
+      long long few = 0;
+      for (BCase* c : G.members) few += c->s2->g.ntiles(0);
+      G.rows = ox2::pick_rows(G.launch2, few);
+      for (BCase* c : G.members) nt[0] += c->s2->g.ntiles(G.rows);
       ntiles.push_back(nt);
       ntiles_les.push_back(nl);
       continue;
@@ -285,16 +289,13 @@ int build_plan(ox_batch* b) {
         for (int d = 0; d < 3; ++d) {
           L.map[d] = b->d_map + map_off[gi] + (size_t)d * n;
           L.ntiles[d] = ntiles[gi][d];
-          L.grid[d] = ntiles[gi][d];
         }
         if (G.les) {
           L.map_les = b->d_map + map_off[gi] + (size_t)3 * n;
           L.ntiles_les = ntiles_les[gi];
-          L.grid_les = ntiles_les[gi];
         }
       } else {
         L.ntiles[0] = ntiles[gi][0];
-        L.grid[0] = ox2::grid2(ntiles[gi][0], G.launch2[st].max_blocks());
       }
       b->launches.push_back(L);
       b->launch_stage.push_back(st);
@@ -326,7 +327,7 @@ int build_plan(ox_batch* b) {
           ox2d_solver* s2 = G.members[m]->s2;
           ox2::write_args2(s2->cfg, s2->g, s2->buf, b->launch_stage[li], tile0,
                            b->h_args + set * b->args_bytes + b->args_off[li] + m * ab);
-          tile0 += s2->ntiles;
+          tile0 += s2->g.ntiles(G.rows);
         }
       }
     }
@@ -438,7 +439,7 @@ void enqueue_step(ox_batch* b, int set) {
       // the boundary fills of this stage's non-periodic cases
       for (; fi < fills.size() && fills[fi].li == li; ++fi) G.ops.bc_after(fills[fi].g, fills[fi].pn, L.stream);
     } else {
-      G.launch2[b->launch_stage[li]].launch(base, L.ncase, L.ntiles[0], L.grid[0], L.stream);
+      G.launch2[b->launch_stage[li]].launch[G.rows](base, L.ncase, L.ntiles[0], L.stream);
     }
   }
 }

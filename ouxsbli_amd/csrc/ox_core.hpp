@@ -81,12 +81,10 @@ struct BatchGroupLaunch {
   const void* args[3];     // device arrays of the per-case sweep descriptors (x, y, z)
   const TileMap* map[3];   // device tile maps (x, y, z)
   int ntiles[3];
-  int grid[3];             // workgroups: the tiles (2-D: a persistent grid)
   int ep;                  // RK epilogue of the stage
   // LES groups: the SGS viscosity
   const TileMap* map_les;
   int ntiles_les;
-  int grid_les;
 };
 
 struct BatchOps {

@@ -26,6 +26,7 @@
 
 #include "ox_physics.hpp"
 #include "ox_types.hpp"
+#include "ox_xcd.hpp"
 
 namespace ox {
 
@@ -69,33 +70,6 @@ template <int ORDER, int VISC, int VO> struct Sten {
   static constexpr int VOFF = VISC ? HW - vwin<VO>() / 2 : 0;
   static constexpr int VH = vcross<VO>() / 2;  // half width of the cross-derivative stencil
 };
-
-// Workgroups are dispatched round-robin over the eight XCDs, and each XCD has
-// its own L2.  Of every 8 * XCD_CHUNK workgroups, those of one XCD take XCD_CHUNK
-// tiles that follow one another, so the tiles whose stencils overlap (neighbours
-// along the second and third launch dimensions) share an L2 instead of fetching
-// the same rows into two, while all XCDs work in one part of the grid and find
-// in the shared cache what the others fetched.  (One run of n / 8 tiles per XCD,
-// for n a multiple of 8 only, was up to 10% slower, us: Hybrid6 LES 192^3 x 405
-// -> 378, y 533 -> 479, z 674 -> 638; SLAU6 NS 256^3 x 735 -> 702, y 778 -> 732, but
-// z 1042 -> 1065; FP32 SLAU6 Euler 256^3 x 296 -> 270; FP32 Roe4 NS 190 x 187 x 181,
-// undivided before, y 145 -> 137, z 271 -> 253; six FP32 requests 138.9 -> 134.2 ms.
-// Chunks of 16 are equal, of 8 and 64 a little slower.)  `few`: a launch of up to
-// 2048 workgroups, which the chip holds at once, is one run per XCD instead; the
-// line sweeps of a lone case take it (FP32 96^3 y, SLAU6 Euler 25.6 -> 24.7 us,
-// KEEP4 NS 17.7 -> 16.9), the x sweep and batches are faster in chunks (FP32 SLAU6
-// Euler 64^3 x 11.4 -> 10.4; the six requests 136.3 -> 133.9 ms).
-// The map is a permutation of [0, n).
-constexpr int XCD_CHUNK = 32;
-__device__ __forceinline__ int xcd_tile(int b, int n, bool few = false) {
-  int base = 0, m = n;
-  if (!few || n > 2048) {
-    base = b / (8 * XCD_CHUNK) * (8 * XCD_CHUNK);
-    m = n - base < 8 * XCD_CHUNK ? n - base : 8 * XCD_CHUNK;
-  }
-  const int c = b - base, x = c & 7, r = m & 7;
-  return base + x * (m >> 3) + (x < r ? x : r) + (c >> 3);
-}
 
 // state index of (i,l,j,k), 0-based: 64-bit, since the state holds five
 // values per cell and a grid of up to 2^31 cells fits one GPU's HBM (the

@@ -125,15 +125,15 @@ template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 void run_stage_batch(const BatchGroupLaunch& L) {
   using A = SweepArgs<R, S>;
   if constexpr (VISC == 2) {
-    k_les_mut_batch<R, S><<<L.grid_les, 256, 0, L.stream>>>((const A*)L.args[0], L.map_les, L.ncase, L.ntiles_les);
+    k_les_mut_batch<R, S><<<L.ntiles_les, 256, 0, L.stream>>>((const A*)L.args[0], L.map_les, L.ncase, L.ntiles_les);
   }
   k_sweep_x_batch<R, S, ORDER, SCHEME, VISC, VO>
-      <<<L.grid[0], 256, 0, L.stream>>>((const A*)L.args[0], L.map[0], L.ncase, L.ntiles[0]);
+      <<<L.ntiles[0], 256, 0, L.stream>>>((const A*)L.args[0], L.map[0], L.ncase, L.ntiles[0]);
   k_sweep_line_batch<R, S, ORDER, SCHEME, VISC, VO, 1, EP_RHS>
-      <<<L.grid[1], line_block(), 0, L.stream>>>((const A*)L.args[1], L.map[1], L.ncase, L.ntiles[1]);
+      <<<L.ntiles[1], line_block(), 0, L.stream>>>((const A*)L.args[1], L.map[1], L.ncase, L.ntiles[1]);
 #define OX_ZB(E)                                         \
   k_sweep_line_batch<R, S, ORDER, SCHEME, VISC, VO, 2, E> \
-      <<<L.grid[2], line_block(), 0, L.stream>>>((const A*)L.args[2], L.map[2], L.ncase, L.ntiles[2])
+      <<<L.ntiles[2], line_block(), 0, L.stream>>>((const A*)L.args[2], L.map[2], L.ncase, L.ntiles[2])
   switch (L.ep) {
     case EP_RK3_S1: OX_ZB(EP_RK3_S1); break;
     case EP_RK3_S23: OX_ZB(EP_RK3_S23); break;
