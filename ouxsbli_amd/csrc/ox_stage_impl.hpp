@@ -112,8 +112,7 @@ void run_stage(Core& C, const double* Qsrc, const StageArgs& sa, double cx, doub
   if (sa.ep != EP_RHS && any_bc(g)) {
     // the case's set_bc on the new state, as ghost primitives (and sensors)
     const Prim<S> Pn = prim_set<S>(C, 1 - C.cur);
-    launch_bc_prims<R, S, ORDER, SCHEME, VISC>(g, Pn, C.stream);
-    launch_bc_sensors<R, S, ORDER, SCHEME>(g, Pn, C.stream);
+    launch_bc_fill<R, S, ORDER, SCHEME>(g, Pn, C.stream);
     prof_mark(C, "bc");
   }
   finish_stage(C, sa);
@@ -154,8 +153,7 @@ void bc_after_erased(const Geom& g, void* const* pn, hipStream_t st) {
   Prim<S> P;
   S** a[kPrimArrays] = {&P.rho, &P.u, &P.v, &P.w, &P.p, &P.s, &P.mut, &P.qc2};
   for (int m = 0; m < kPrimArrays; ++m) *a[m] = (S*)pn[m];
-  launch_bc_prims<R, S, ORDER, SCHEME, VISC>(g, P, st);
-  launch_bc_sensors<R, S, ORDER, SCHEME>(g, P, st);
+  launch_bc_fill<R, S, ORDER, SCHEME>(g, P, st);
 }
 
 // Workgroups of k_sweep_line one compute unit holds, asked once per kernel.
