@@ -67,7 +67,7 @@ def kernel_model(spec, ops):
 # the kernel sources they were measured on: a kernel change makes them stale,
 # and the bench line then reports traffic null.
 TRAFFIC_FILE = ROOT / "ouxsbli_amd" / "flops" / "traffic.json"
-KERNEL_SOURCES = ("ox_kernels.hpp", "ox_physics.hpp", "ox_stage_impl.hpp", "ox_types.hpp", "ox_core.hpp",
+KERNEL_SOURCES = ("ox_kernels.hpp", "ox_physics.hpp", "ox_stage_impl.hpp", "ox_types.hpp", "ox_core.hpp", "ox_xcd.hpp",
                   "ox_fp64.hip")
 
 

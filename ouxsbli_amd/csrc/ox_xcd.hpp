@@ -14,7 +14,8 @@ namespace ox {
 // for n a multiple of 8 only, was up to 10% slower, us: Hybrid6 LES 192^3 x 405
 // -> 378, y 533 -> 479, z 674 -> 638; SLAU6 NS 256^3 x 735 -> 702, y 778 -> 732, but
 // z 1042 -> 1065; FP32 SLAU6 Euler 256^3 x 296 -> 270; FP32 Roe4 NS 190 x 187 x 181,
-// undivided before, y 145 -> 137, z 271 -> 253; six FP32 requests 138.9 -> 134.2 ms.
+// undivided before, y 145 -> 137, z 271 -> 253; six FP32 requests 138.9 -> 133.9 ms; over
+// the 256^3 Taylor-Green runs the step is the same within 0.6%.
 // Chunks of 16 are equal, of 8 and 64 a little slower.)  `few`: a launch of up to
 // 2048 workgroups, which the chip holds at once, is one run per XCD instead; the
 // line sweeps of a lone case take it (FP32 96^3 y, SLAU6 Euler 25.6 -> 24.7 us,
