@@ -226,7 +226,7 @@ def batched_os_leg(ncase, steps, unbatched_steps, cpu_seconds):
     nx-2 ~ U{128..512}, ny-2 ~ U{64..256}, Mach 2, deflection ~ U(4, 12) deg
     (seeded), Rankine-Hugoniot state on the top boundary, Roe + MUSCL (ORDER 6,
     hybrid limiter), RK3, FP32 bulk, `steps` steps each, all resident and
-    advanced together: one persistent launch per RK stage over the tiles of
+    advanced together: one launch per RK stage over the tiles of
     all cases, replayed from a HIP graph.  Timed beside: the FP64 plain form
     of the same batch, and the FP32 cases advanced one by one (one launch per
     stage per case), in both forms."""
@@ -236,7 +236,7 @@ def batched_os_leg(ncase, steps, unbatched_steps, cpu_seconds):
     from ouxsbli_amd.solver2d import Solver2D
     out = {"workload": f"{ncase} batched 2-D oblique-shock reflections, interior 128..512 x 64..256, M 2, "
                        "theta U(4,12) deg, Roe + MUSCL ORDER 6 hybrid limiter, RK3, "
-                       f"{steps} steps each, one persistent launch per stage with HIP graph replay",
+                       f"{steps} steps each, one launch per stage with HIP graph replay",
            "cases": ncase, "steps": steps}
     res = {}
     for prec in ("fp32_bulk", "fp64"):

@@ -1,7 +1,7 @@
 """Python handle over the batch engine of include/ouxsbli.h (ox_batch_*).
 
 Many cases are resident on the GPU at once; every ``step()`` advances all of
-them by one RK step, with one persistent launch per sweep and RK stage for
+them by one RK step, with one launch per sweep and RK stage for
 each group of cases that share a kernel specialisation, replayed from a
 captured HIP graph while the set of cases is unchanged.  Cases join with
 ``admit`` (refused with ``Busy`` while they do not fit in the free slots or
