@@ -166,6 +166,11 @@ __global__ void k_diag_merge(const double* __restrict__ part, int nb, double* __
 
 int ox_fail(int code, const std::string& msg) {
   g_err = msg;
+  // HIP keeps an error until it is asked for: one that is reported here must not
+  // come back from the launch check of a later call, which may be on another,
+  // healthy handle (a result that cannot be page-locked is an ordinary array, and
+  // an admission that runs out of memory is tried again)
+  if (code == OX_EDEVICE || code == OX_ENOMEM) (void)hipGetLastError();
   return code;
 }
 
