@@ -50,6 +50,7 @@ UNITS = {
     "ox_fp32.hip": FP32_BULK,
     "ox_fp32_batch.hip": FP32_BULK,
     "ox2d_capi.hip": ["-ffp-contract=off"],
+    "ox_hostcopy.hip": ["-ffp-contract=off"],
     "ox_ic.hip": ["-ffp-contract=off"],
     "ox2d_fp64.hip": ["-ffp-contract=off"],
     "ox2d_fp32.hip": FP32_BULK,

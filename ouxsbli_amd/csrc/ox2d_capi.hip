@@ -145,9 +145,7 @@ int ox2d_get_state(ox2d_solver* s, double* Q) {
   // data between steps (every stage writes all points of its output)
   ox2::k2d_scale<<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->buf[0], s->buf[1], n, s->g.J, 0);
   OX_HIP(hipGetLastError());
-  OX_HIP(hipMemcpyAsync(Q, s->buf[1], n * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-  OX_HIP(hipStreamSynchronize(s->stream));
-  return OX_OK;
+  return copy_to_host(s->cfg.device, Q, s->buf[1], n * sizeof(double), s->stream);
 }
 
 int ox2d_step(ox2d_solver* s, int32_t nsteps) {

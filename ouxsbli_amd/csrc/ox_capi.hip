@@ -486,9 +486,7 @@ int ox_get_qj(ox_solver* s, double* QJ) {
   if (!s || !QJ) return ox_fail(OX_EINVAL, "null argument");
   OX_HIP(hipSetDevice(s->C.cfg.device));
   const size_t n = state_elems(s->C.g);
-  OX_HIP(hipMemcpyAsync(QJ, s->QJ, n * sizeof(double), hipMemcpyDeviceToHost, s->C.stream));
-  OX_HIP(hipStreamSynchronize(s->C.stream));
-  return OX_OK;
+  return copy_to_host(s->C.cfg.device, QJ, s->QJ, n * sizeof(double), s->C.stream);
 }
 
 int ox_set_state(ox_solver* s, const double* Q) {
@@ -512,9 +510,7 @@ int ox_get_state(ox_solver* s, double* Q) {
   ox::k_scale_to<<<(unsigned)((n + 255) / 256), 256, 0, s->C.stream>>>(s->QJ, s->QJ2, n, s->C.g.jac);
   OX_HIP(hipGetLastError());
   if (s->C.prim_for == s->QJ2) s->C.prim_for = nullptr;
-  OX_HIP(hipMemcpyAsync(Q, s->QJ2, n * sizeof(double), hipMemcpyDeviceToHost, s->C.stream));
-  OX_HIP(hipStreamSynchronize(s->C.stream));
-  return OX_OK;
+  return copy_to_host(s->C.cfg.device, Q, s->QJ2, n * sizeof(double), s->C.stream);
 }
 
 int ox_step(ox_solver* s, int32_t nsteps) {
@@ -572,9 +568,7 @@ int ox_rhs(ox_solver* s, double* R) {
   ox::StageArgs sa{s->QJ, s->QJ2, s->Rs, 0, 0, 0, ox::EP_RHS};
   s->stage(s->C, s->QJ, sa, g.a_yz, g.a_zx, g.a_xy);
   OX_HIP(hipGetLastError());
-  OX_HIP(hipMemcpyAsync(R, s->QJ2, n * sizeof(double), hipMemcpyDeviceToHost, s->C.stream));
-  OX_HIP(hipStreamSynchronize(s->C.stream));
-  return OX_OK;
+  return copy_to_host(s->C.cfg.device, R, s->QJ2, n * sizeof(double), s->C.stream);
 }
 
 int ox_diagnostics(ox_solver* s, ox_diag* out) {

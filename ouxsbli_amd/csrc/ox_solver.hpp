@@ -57,5 +57,9 @@ void rk_stage(ox_solver* s, int st, const double** Qsrc, ox::StageArgs* sa, doub
 // each stream of the process, which made retiring one of 64 cases take 0.9 ms.
 int solver_create(const ox_config* cfg, hipStream_t shared, ox_solver** out);
 
+// Copies a result of `bytes` bytes, which work queued on `stream` of device `device`
+// may still be writing, into host memory of any kind and waits for it.
+int copy_to_host(int device, void* dst, const void* src, size_t bytes, hipStream_t stream);
+
 // Device bytes a handle with this configuration allocates.
 size_t solver_footprint(const ox_config& c);

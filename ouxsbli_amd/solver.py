@@ -12,7 +12,6 @@ import ctypes
 import numpy as np
 
 from . import _abi, _native
-from .batch import pinned_pool
 from .cases import CaseSpec
 
 
@@ -70,10 +69,7 @@ class Solver:
         _native.check(self._lib.ox_init_state(self._h, ctypes.byref(ic)))
 
     def get_state(self) -> np.ndarray:
-        """The physical state, on a page-locked buffer of the process's pool (a
-        copy into ordinary memory is staged: 68 ms against 13 for the 720 MB
-        of 256^3)."""
-        Q = pinned_pool().array(self.spec.state_shape())
+        Q = np.empty(self.spec.state_shape())
         _native.check(self._lib.ox_get_state(self._h, _dp(Q)))
         return Q
 
@@ -82,7 +78,7 @@ class Solver:
         _native.check(self._lib.ox_set_qj(self._h, _dp(QJ)))
 
     def get_qj(self) -> np.ndarray:
-        QJ = pinned_pool().array(self.spec.state_shape())
+        QJ = np.empty(self.spec.state_shape())
         _native.check(self._lib.ox_get_qj(self._h, _dp(QJ)))
         return QJ
 
@@ -95,7 +91,7 @@ class Solver:
         return ms.value
 
     def rhs(self) -> np.ndarray:
-        R = pinned_pool().array(self.spec.state_shape())
+        R = np.empty(self.spec.state_shape())
         _native.check(self._lib.ox_rhs(self._h, _dp(R)))
         return R
 

@@ -13,7 +13,6 @@ import ctypes
 import numpy as np
 
 from . import _native
-from .batch import pinned_pool
 from .cases2d import CaseSpec2D
 
 
@@ -62,7 +61,7 @@ class Solver2D:
         _native.check(self._lib.ox2d_init_state(self._h))
 
     def get_state(self) -> np.ndarray:
-        Q = pinned_pool().array(self.spec.state_shape())
+        Q = np.empty(self.spec.state_shape(), dtype=np.float64)
         _native.check(self._lib.ox2d_get_state(self._h, _dp(Q)))
         return Q
 
