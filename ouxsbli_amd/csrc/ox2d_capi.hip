@@ -19,7 +19,7 @@
 namespace ox2 {
 // dst = src / J (divide) or J * src over n values; dst may be src.
 __global__ __launch_bounds__(256) void k2d_scale(const double* src, double* dst, size_t n, double J, int divide) {
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const size_t t = (size_t)ox::launch_block() * 256 + threadIdx.x;
   if (t < n) dst[t] = divide ? src[t] / J : J * src[t];
 }
 }  // namespace ox2
@@ -131,7 +131,7 @@ int ox2d_set_state(ox2d_solver* s, const double* Q) {
   const size_t n = state2_elems(s->cfg);
   OX_HIP(hipMemcpyAsync(s->buf[0], Q, n * sizeof(double), hipMemcpyHostToDevice, s->stream));
   // pre_calc: QJ = Q / J
-  ox2::k2d_scale<<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->buf[0], s->buf[0], n, s->g.J, 1);
+  ox2::k2d_scale<<<ox::launch_grid((n + 255) / 256), 256, 0, s->stream>>>(s->buf[0], s->buf[0], n, s->g.J, 1);
   OX_HIP(hipGetLastError());
   OX_HIP(hipStreamSynchronize(s->stream));
   return OX_OK;
@@ -143,7 +143,7 @@ int ox2d_get_state(ox2d_solver* s, double* Q) {
   const size_t n = state2_elems(s->cfg);
   // main.f90:84: Q = J * QJ, into the first stage's buffer, which holds no live
   // data between steps (every stage writes all points of its output)
-  ox2::k2d_scale<<<(unsigned)((n + 255) / 256), 256, 0, s->stream>>>(s->buf[0], s->buf[1], n, s->g.J, 0);
+  ox2::k2d_scale<<<ox::launch_grid((n + 255) / 256), 256, 0, s->stream>>>(s->buf[0], s->buf[1], n, s->g.J, 0);
   OX_HIP(hipGetLastError());
   return copy_to_host(s->cfg.device, Q, s->buf[1], n * sizeof(double), s->stream);
 }

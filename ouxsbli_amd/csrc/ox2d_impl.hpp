@@ -9,7 +9,7 @@ namespace ox2 {
 
 template <class R, int ORDER, int SCHEME, int EP, int ROW>
 void launch2(const void* args, int ncase, int ntiles, hipStream_t stream) {
-  k2d_stage<R, ORDER, SCHEME, EP, ROW><<<ntiles, LANES, 0, stream>>>((const Args2<R>*)args, ncase);
+  k2d_stage<R, ORDER, SCHEME, EP, ROW><<<ox::launch_grid(ntiles), LANES, 0, stream>>>((const Args2<R>*)args, ncase, ntiles);
 }
 
 template <class R, int ORDER, int SCHEME, int EP> int few_tiles() {

@@ -360,9 +360,11 @@ __device__ __forceinline__ int find_case2(const Args2<R>* __restrict__ args, int
 // n-th tile, took 52 us for an FP32 stage of 2047 x 1023 where this takes 46, and 51
 // ms for 150 steps of 64 FP32 cases of 257 x 129 where this takes 45.)
 template <class R, int ORDER, int SCHEME, int EP, int ROW>
-__global__ __launch_bounds__(LANES) void k2d_stage(const Args2<R>* __restrict__ args, int ncase) {
+__global__ __launch_bounds__(LANES) void k2d_stage(const Args2<R>* __restrict__ args, int ncase, int ntiles) {
   __shared__ Tile2<R, ORDER, ROW> T;
-  const int t = ox::xcd_tile(blockIdx.x, gridDim.x, true);
+  const unsigned b = ox::launch_block();
+  if (b >= (unsigned)ntiles) return;
+  const int t = ox::xcd_tile(b, ntiles, true);
   const Args2<R>& a = args[find_case2(args, ncase, t)];
   const int local = t - a.tile0;
   stage_tile<R, ORDER, SCHEME, EP, ROW>(a, local % a.nbx, local / a.nbx, T);

@@ -1069,7 +1069,9 @@ template <class R, class S, int ORDER, int SCHEME, int VISC, int VO>
 __global__ __launch_bounds__(256) void k_sweep_x_batch(const SweepArgs<R, S>* __restrict__ cases,
                                                        const TileMap* __restrict__ map, int ncase, int ntiles) {
   __shared__ XRunTile<R, ORDER, SCHEME, VISC, VO> lds;
-  const int t = xcd_tile(blockIdx.x, ntiles), ci = find_case(map, ncase, t);
+  const unsigned b = launch_block();
+  if (b >= (unsigned)ntiles) return;
+  const int t = xcd_tile(b, ntiles), ci = find_case(map, ncase, t);
   sweep_x_run<R, S, ORDER, SCHEME, VISC, VO>(cases[ci], t - map[ci].start, lds);
 }
 

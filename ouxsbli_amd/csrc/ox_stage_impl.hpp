@@ -127,7 +127,7 @@ void run_stage_batch(const BatchGroupLaunch& L) {
     k_les_mut_batch<R, S><<<L.ntiles_les, 256, 0, L.stream>>>((const A*)L.args[0], L.map_les, L.ncase, L.ntiles_les);
   }
   k_sweep_x_batch<R, S, ORDER, SCHEME, VISC, VO>
-      <<<L.ntiles[0], 256, 0, L.stream>>>((const A*)L.args[0], L.map[0], L.ncase, L.ntiles[0]);
+      <<<launch_grid(L.ntiles[0]), 256, 0, L.stream>>>((const A*)L.args[0], L.map[0], L.ncase, L.ntiles[0]);
   k_sweep_line_batch<R, S, ORDER, SCHEME, VISC, VO, 1, EP_RHS>
       <<<L.ntiles[1], line_block(), 0, L.stream>>>((const A*)L.args[1], L.map[1], L.ncase, L.ntiles[1]);
 #define OX_ZB(E)                                         \

@@ -1,9 +1,20 @@
-// ox_xcd.hpp -- which tile a workgroup takes: the deal over the XCDs.
+// ox_xcd.hpp -- which tile a workgroup takes: launches of any length, and the deal
+// over the XCDs.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 namespace ox {
+
+// The grid of a launch of n workgroups of up to 512 lanes, and a workgroup's number
+// in it (not below n in the last row: nothing to do).  HIP refuses 2^32 or more work
+// items in one dimension, which the tiles of thin grids and of long batches reach
+// (8 x 2^27 points in 2-D: 19 million tiles), so longer launches are folded.
+constexpr int LAUNCH_ROW = 1 << 22;
+__host__ inline dim3 launch_grid(long long n) {
+  return n <= LAUNCH_ROW ? dim3((unsigned)n) : dim3(LAUNCH_ROW, (unsigned)((n + LAUNCH_ROW - 1) / LAUNCH_ROW));
+}
+__device__ __forceinline__ unsigned launch_block() { return blockIdx.x + gridDim.x * blockIdx.y; }
 
 // Workgroups are dispatched round-robin over the eight XCDs, and each XCD has
 // its own L2.  Of every 8 * XCD_CHUNK workgroups, those of one XCD take XCD_CHUNK
