@@ -1206,7 +1206,10 @@ inline int pick_lseg(const LineWork* p, int n, int occ, int cus) {
 // four waves as they are, and their ring was slower (SLAU6 NS at 128^3: y 58 ->
 // 62, z 87 -> 88 us).  LES stays in registers at one wave: with its ring (mt and H
 // as well) the FP64 z sweep spilled and took 780 us where it takes 691 (Hybrid6
-// at 192^3).
+// at 192^3).  Built without the memory-clause scheduler that the FP64 units use, that
+// LES ring ended in an illegal memory access (Hybrid6 LES, FP64, 192^3).  Its cause is
+// not known: neither ring's indices leave their arrays, nor is a slot read before it
+// is written, in a host build with every array checked.  So the form is closed.
 template <class R, int SCHEME, int VISC> constexpr int ring_fields() {
   return VISC != 1 || sizeof(R) != 8 ? 0 : kUsesT<SCHEME> ? 5 : 6;  // d1..d4, mu[, T]
 }
@@ -1281,6 +1284,7 @@ __device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx
   };
   using RC = RawCell<S, VISC, VO>;
   constexpr bool RING = ring_fields<R, SCHEME, VISC>() > 0;
+  static_assert(!(RING && VISC == 2), "no LES ring before the cause of its memory access fault is known");
   R* mine = ring + threadIdx.x + LINE_X * threadIdx.y;
   CD win[St::SW];
 #pragma unroll
