@@ -50,11 +50,13 @@ int validate2(const ox2d_config& c) {
 }
 
 size_t state2_elems(const ox2d_config& c) { return (size_t)c.nx * 4 * (size_t)c.ny; }
+// bytes from one of the three states to the next, which starts at a multiple of 256
+size_t state2_stride(const ox2d_config& c) { return (state2_elems(c) * sizeof(double) + 255) & ~(size_t)255; }
 
 }  // namespace
 
 size_t solver2d_footprint(const ox2d_config& c) {
-  return 3 * state2_elems(c) * sizeof(double) + 3 * ox2::args2_bytes(c.precision);
+  return 3 * state2_stride(c) + 3 * ox2::args2_bytes(c.precision);
 }
 
 extern "C" {
@@ -105,9 +107,9 @@ int solver2d_create(const ox2d_config* cfg, hipStream_t shared, ox2d_solver** ou
       hipEventCreate(&s->ev0) != hipSuccess || hipEventCreate(&s->ev1) != hipSuccess)
     return fail(OX_EDEVICE, "stream/event creation failed");
   s->stream = shared ? shared : s->own_stream;
-  const size_t bytes = (state2_elems(*cfg) * sizeof(double) + 255) & ~(size_t)255;
+  const size_t bytes = state2_stride(*cfg);
   s->args_bytes = ox2::args2_bytes(cfg->precision);
-  if (hipMalloc(&s->slab, 3 * bytes + 3 * s->args_bytes) != hipSuccess) return fail(OX_ENOMEM, "device allocation failed");
+  if (hipMalloc(&s->slab, solver2d_footprint(*cfg)) != hipSuccess) return fail(OX_ENOMEM, "device allocation failed");
   if (hipMemsetAsync(s->slab, 0, 3 * bytes, s->stream) != hipSuccess) return fail(OX_EDEVICE, "hipMemsetAsync failed");
   for (int k = 0; k < 3; ++k) s->buf[k] = (double*)(s->slab + k * bytes);
   s->d_args = s->slab + 3 * bytes;

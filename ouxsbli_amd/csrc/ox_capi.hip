@@ -214,16 +214,44 @@ void rk_stage(ox_solver* s, int st, const double** Qsrc, ox::StageArgs* sa, doub
   }
 }
 
-size_t solver_footprint(const ox_config& c) {
-  const size_t ns = (size_t)c.nx * 5 * c.ny * c.nz, nc = (size_t)c.nx * c.ny * c.nz;
-  const size_t pe = c.precision == OX_PREC_FP64 ? sizeof(double) : sizeof(float);
-  // rho,u,v,w,p,sensor (+mut,qc2 for LES); the sweeps form T and mu
-  const size_t nprim = 6 + (c.visc == OX_VISC_LES ? 2 : 0);
-  size_t b = 2 * ns * sizeof(double) + ns * pe + 2 * nprim * nc * pe;  // QJ, QJ2, Racc, two primitive sets
-  if (c.rk == 4) b += ns * sizeof(double);                             // Rs
-  b += 4096 * (2 * ox::DIAG_NQ + 1) * sizeof(double);                  // reduction partials
-  return b;
-}
+namespace {
+
+// Where the arrays of a handle lie in its one allocation, each from a multiple of
+// 256 bytes on.
+struct Layout {
+  size_t qj, qj2, racc, rs, prim[2][ox::kPrimArrays], scratch;
+  int nprim;
+  size_t cleared;  // everything before the reduction partials starts as zero
+  size_t scratch_bytes, bytes;
+
+  explicit Layout(const ox_config& c) {
+    const size_t nc = (size_t)c.nx * c.ny * c.nz, ns = 5 * nc;
+    const size_t pe = c.precision == OX_PREC_FP64 ? sizeof(double) : sizeof(float);
+    bytes = 0;
+    qj = place(ns * sizeof(double));
+    qj2 = place(ns * sizeof(double));
+    racc = place(ns * pe);
+    rs = place(c.rk == 4 ? ns * sizeof(double) : 0);
+    // rho,u,v,w,p,sensor (+mut,qc2 for LES); the sweeps form T and mu
+    nprim = c.visc == OX_VISC_LES ? 8 : 6;
+    for (int set = 0; set < 2; ++set)
+      for (int m = 0; m < nprim; ++m) prim[set][m] = place(nc * pe);
+    cleared = bytes;
+    scratch_bytes = 4096 * (2 * ox::DIAG_NQ + 1) * sizeof(double);
+    scratch = place(scratch_bytes);
+  }
+
+ private:
+  size_t place(size_t n) {
+    const size_t at = bytes;
+    bytes += (n + 255) & ~(size_t)255;
+    return at;
+  }
+};
+
+}  // namespace
+
+size_t solver_footprint(const ox_config& c) { return Layout(c).bytes; }
 
 namespace {
 
@@ -389,41 +417,27 @@ int solver_create(const ox_config* cfg, hipStream_t shared, ox_solver** out) {
     return ox_fail(OX_EDEVICE, std::string("hipSetDevice: ") + hipGetErrorString(e));
   }
   ox::solo_segments(C.g, ops, C.lseg);
-  const size_t ns = state_elems(C.g), nc = cell_elems(C.g);
-  const size_t pe = cfg->precision == OX_PREC_FP64 ? sizeof(double) : sizeof(float);
   bool ok = shared || hipStreamCreateWithFlags(&s->own_stream, hipStreamNonBlocking) == hipSuccess;
   C.stream = shared ? shared : s->own_stream;
   // every array of the handle in one allocation: a hipFree of more than a few
   // MB costs about 0.1 ms, whatever its size
-  const int nprim = cfg->visc == OX_VISC_LES ? 8 : 6;  // arrays 6 and 7 (mut, qc2) only for LES
-  s->scratch_bytes = 4096 * (2 * ox::DIAG_NQ + 1) * sizeof(double);
-  size_t bytes = 0;
-  auto place = [&bytes](size_t n) {
-    const size_t at = bytes;
-    bytes += (n + 255) & ~(size_t)255;
-    return at;
-  };
-  const size_t at_qj = place(ns * sizeof(double)), at_qj2 = place(ns * sizeof(double)), at_racc = place(ns * pe);
-  const size_t at_rs = cfg->rk == 4 ? place(ns * sizeof(double)) : 0;
-  size_t at_prim[2][8];
-  for (int set = 0; set < 2; ++set)
-    for (int m = 0; m < nprim; ++m) at_prim[set][m] = place(nc * pe);
-  const size_t cleared = bytes, at_scratch = place(s->scratch_bytes);
-  ok = ok && hipMalloc(&s->slab, bytes) == hipSuccess;
+  const Layout at(*cfg);
+  ok = ok && hipMalloc(&s->slab, at.bytes) == hipSuccess;
   ok = ok && hipEventCreate(&s->ev0) == hipSuccess && hipEventCreate(&s->ev1) == hipSuccess;
   if (!ok) {
     destroy(s);
     return ox_fail(OX_ENOMEM, "device allocation failed");
   }
-  s->QJ = (double*)(s->slab + at_qj);
-  s->QJ2 = (double*)(s->slab + at_qj2);
-  C.Racc = s->slab + at_racc;
-  if (cfg->rk == 4) s->Rs = (double*)(s->slab + at_rs);
+  s->QJ = (double*)(s->slab + at.qj);
+  s->QJ2 = (double*)(s->slab + at.qj2);
+  C.Racc = s->slab + at.racc;
+  if (cfg->rk == 4) s->Rs = (double*)(s->slab + at.rs);
   for (int set = 0; set < 2; ++set)
-    for (int m = 0; m < nprim; ++m) C.prim[set][m] = s->slab + at_prim[set][m];
-  s->scratch = (double*)(s->slab + at_scratch);
+    for (int m = 0; m < at.nprim; ++m) C.prim[set][m] = s->slab + at.prim[set][m];
+  s->scratch = (double*)(s->slab + at.scratch);
+  s->scratch_bytes = at.scratch_bytes;
   // Zero everything once: ghost layers of QJ2 and the accumulators start defined.
-  ok = hipMemsetAsync(s->slab, 0, cleared, C.stream) == hipSuccess;
+  ok = hipMemsetAsync(s->slab, 0, at.cleared, C.stream) == hipSuccess;
   ok = ok && hipStreamSynchronize(C.stream) == hipSuccess;
   if (!ok) {
     destroy(s);
