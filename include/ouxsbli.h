@@ -256,7 +256,8 @@ typedef struct ox_batch_config {
   int32_t device;
   int32_t max_cases;     /* resident cases at most (slots)                    */
   int32_t use_graph;     /* replay each step from a captured HIP graph        */
-  int32_t autotune;      /* tune segment lengths per (specialisation, grid)   */
+  int32_t autotune;      /* tune the segment lengths of a case that is admitted
+                            into a group of its own, per (specialisation, grid) */
   int32_t pad;
   uint64_t hbm_budget;   /* device bytes the resident cases may hold          */
 } ox_batch_config;
@@ -285,7 +286,9 @@ int ox_batch_admit(ox_batch* b, const ox_config* cfg, const double* Q, int32_t n
 
 /* Fills the engine's segment-length cache for cases of this configuration
  * (grid and specialisation) by tuning on the state Q, without admitting
- * anything: lets a server tune ahead of a request stream. */
+ * anything: lets a server tune ahead of a request stream.  Cached lengths serve a
+ * case while it is the only one of its group; cases that share launches take
+ * lengths chosen by rule for the tiles of all of them. */
 int ox_batch_tune(ox_batch* b, const ox_config* cfg, const double* Q);
 
 /* One RK step of every active case (all groups), then blocks until it has

@@ -183,8 +183,8 @@ class Batch:
         return cid.value
 
     def tune(self, spec: CaseSpec, Q: np.ndarray) -> None:
-        """Tunes (and caches) the segment lengths of cases like ``spec``
-        without admitting anything."""
+        """Tunes (and caches) the segment lengths of cases like ``spec``, for
+        when they are alone in their group, without admitting anything."""
         Q = np.ascontiguousarray(Q, dtype=np.float64)
         cfg = spec.to_ox()
         _native.check(self._lib.ox_batch_tune(self._h, ctypes.byref(cfg),

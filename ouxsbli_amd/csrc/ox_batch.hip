@@ -68,6 +68,17 @@ struct BCase {
   int stages() const { return s2 ? 3 : s->C.cfg.rk; }
 };
 
+// Cases of one key share launches: dimension, precision, specialisation, RK scheme.
+using GroupKey = std::array<int, 4>;
+GroupKey group_key(const ox_solver* s) {
+  const ox::Core& C = s->C;
+  return {3, (int)C.cfg.precision, ox::stage_key(C.cfg.order, C.cfg.scheme, C.cfg.visc, C.vorder), (int)C.cfg.rk};
+}
+GroupKey group_key(const BCase* c) {
+  if (c->s) return group_key(c->s);
+  return {2, (int)c->s2->cfg.precision, ox2::key2(c->s2->cfg.order, c->s2->cfg.scheme), 3};
+}
+
 // Cases sharing a kernel specialisation.  3-D groups launch three sweeps per
 // stage (LES groups first the SGS viscosity);
 // 2-D groups one fused stage kernel (launch2[stage]).
@@ -157,19 +168,7 @@ int build_plan(ox_batch* b) {
   b->groups.clear();
   for (auto& up : b->active) {
     BCase* c = up.get();
-    const int dim = c->dim();
-    int prec, key, rk;
-    if (dim == 3) {
-      const ox::Core& C = c->s->C;
-      prec = C.cfg.precision;
-      key = ox::stage_key(C.cfg.order, C.cfg.scheme, C.cfg.visc, C.vorder);
-      rk = C.cfg.rk;
-    } else {
-      const ox2d_config& k2 = c->s2->cfg;
-      prec = k2.precision;
-      key = ox2::key2(k2.order, k2.scheme);
-      rk = 3;
-    }
+    const auto [dim, prec, key, rk] = group_key(c);
     int gi = -1;
     for (size_t g = 0; g < b->groups.size(); ++g) {
       const BGroup& G = b->groups[g];
@@ -407,8 +406,11 @@ void advance_parity(ox_batch* b, int steps) {
   }
 }
 
-// Segment lengths of a case from the engine's cache, tuning on a miss.
-int tune_case(ox_batch* b, ox_solver* s) {
+// Segment lengths of a case on its own: those that the engine has measured for its
+// kind, measured now if there are none yet and the case would use them (a case that
+// shares launches gets the rule's lengths for all their tiles; measuring ten or so
+// lengths for it, four right-hand sides each, would only delay its admission).
+int tune_case(ox_batch* b, ox_solver* s, bool measure) {
   const ox_config& cfg = s->C.cfg;
   const auto key = std::make_tuple((int)cfg.precision, ox::stage_key(cfg.order, cfg.scheme, cfg.visc, s->C.vorder),
                                    (int)cfg.nx, (int)cfg.ny, (int)cfg.nz);
@@ -418,6 +420,7 @@ int tune_case(ox_batch* b, ox_solver* s) {
     s->C.lseg[1] = ox::clamp_lseg(s->C.g, 2, it->second.second);
     return OX_OK;
   }
+  if (!measure) return OX_OK;  // by rule, as solver_create set them
   int32_t ly, lz;
   const int rc = ox_autotune(s, &ly, &lz);  // leaves the state unchanged
   if (rc == OX_OK) b->tuned[key] = {ly, lz};
@@ -468,7 +471,11 @@ int admit3d(ox_batch* b, const ox_config* cfg, Init init, int32_t nsteps, int64_
   int rc = solver_create(cfg, b->stream, &s);
   if (rc != OX_OK) return rc;
   rc = init(s);
-  if (rc == OX_OK && b->cfg.autotune) rc = tune_case(b, s);
+  if (rc == OX_OK && b->cfg.autotune) {
+    bool shares = false;
+    for (const auto& c : b->active) shares = shares || group_key(c.get()) == group_key(s);
+    rc = tune_case(b, s, !shares);
+  }
   if (rc != OX_OK) {
     ox_destroy(s);
     return rc;
@@ -619,7 +626,7 @@ int ox_batch_tune(ox_batch* b, const ox_config* cfg, const double* Q) {
   int rc = ox_create(cfg, &s);
   if (rc != OX_OK) return rc;
   rc = ox_set_state(s, Q);
-  if (rc == OX_OK) rc = tune_case(b, s);
+  if (rc == OX_OK) rc = tune_case(b, s, true);
   ox_destroy(s);
   return rc;
 }
@@ -769,16 +776,9 @@ int ox_batch_query(ox_batch* b, ox_batch_stats* out) {
   out->done = (int32_t)b->done.size();
   int ng = 0;
   {
-    std::vector<std::tuple<int, int, int, int>> seen;
+    std::vector<GroupKey> seen;
     for (auto& c : b->active) {
-      std::tuple<int, int, int, int> t;
-      if (c->s2) {
-        t = std::make_tuple(2, (int)c->s2->cfg.precision, ox2::key2(c->s2->cfg.order, c->s2->cfg.scheme), 3);
-      } else {
-        const ox::Core& C = c->s->C;
-        t = std::make_tuple(3, (int)C.cfg.precision, ox::stage_key(C.cfg.order, C.cfg.scheme, C.cfg.visc, C.vorder),
-                            (int)C.cfg.rk);
-      }
+      const GroupKey t = group_key(c.get());
       if (std::find(seen.begin(), seen.end(), t) == seen.end()) seen.push_back(t);
     }
     ng = (int)seen.size();

@@ -137,11 +137,12 @@ def serve(requests: List[Request], hbm_budget: int, max_cases: int = 64, use_gra
     """Runs the stream to completion and returns the per-request timings.
 
     With ``autotune`` the engine tunes a shape's segment lengths when it first
-    admits it, inside that request's latency, and keeps the result for later
-    requests of the same shape (an engine passed in as ``batch`` keeps what
-    earlier streams tuned).  ``pretune`` instead fills the cache for every
-    shape of the stream before the clock starts, which a live server cannot
-    do; it is off by default.  The report's engine statistics cover this
+    admits it into a group of its own, inside that request's latency, and keeps
+    the result for later requests of the same shape (an engine passed in as
+    ``batch`` keeps what earlier streams tuned); requests that share launches
+    take lengths chosen by rule for all of them.  ``pretune`` instead fills the
+    cache for every shape of the stream before the clock starts, which a live
+    server cannot do; it is off by default.  The report's engine statistics cover this
     stream only."""
     own = batch is None
     if own:
