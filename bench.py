@@ -338,7 +338,8 @@ def serving_leg(n_requests, fp64_value):
     initial state built on the device when it is admitted.
 
     - cold: a fresh engine; segment lengths are tuned when a shape is first
-      admitted, inside that request's latency;
+      admitted into a group of its own, inside that request's latency (cases
+      that share launches take lengths chosen by rule for all of them);
     - warm: an engine that served an earlier stream (another seed, 2 steps per
       request) keeps its tuned shapes, as a running server does; shapes it
       has not seen are tuned on admission as in the cold run;
@@ -353,7 +354,7 @@ def serving_leg(n_requests, fp64_value):
            "hbm_budget_GiB": SERVE_BUDGET >> 30, "slots": SERVE_SLOTS}
     cold = _serve_once(n_requests, "fp32_bulk", seed)
     out.update(cold)
-    out["tuning"] = "cold: each new shape tuned at admission, inside latency"
+    out["tuning"] = "cold: a new shape is tuned when it is admitted into a group of its own, inside latency"
     warm = {}
     for prec in ("fp32_bulk", "fp64"):
         with Batch(SERVE_BUDGET, max_cases=SERVE_SLOTS, use_graph=True, autotune=True) as b:

@@ -242,10 +242,11 @@ int ox_set_segments(ox_solver* s, int32_t lseg_y, int32_t lseg_z);
  * that share a kernel specialisation and RK scheme form a group; one RK stage
  * of a group is one launch per sweep over the tiles of all its cases (LES
  * groups first run the SGS viscosity, calc_les.f90:96-125, with its ghost
- * copy, set_bc_common.f90:296-335, as a launch over the same cases), and one step of the whole batch is replayed from a captured HIP
- * graph while the set of cases does not change.  Cases join (ox_batch_admit)
- * and leave (when their step count is reached) between steps.  The reference
- * has no counterpart: it runs one case per `mpirun` (ouxsbli/case.py:180-201).
+ * copy, set_bc_common.f90:296-335, as a launch over the same cases), and one
+ * step of the whole batch is replayed from a captured HIP graph while the set
+ * of cases does not change.  Cases join (ox_batch_admit) and leave (when their
+ * step count is reached) between steps.  The reference has no counterpart: it
+ * runs one case per `mpirun` (ouxsbli/case.py:180-201).
  * Each case's result is bit-identical to advancing it alone with ox_step.
  * A batch is driven from one host thread.
  * ------------------------------------------------------------------------- */

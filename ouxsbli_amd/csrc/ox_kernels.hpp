@@ -669,8 +669,9 @@ __device__ __forceinline__ R ducros_x(const Geom& g, const DucrosPart<R>& d, R u
 // the schemes that read the Ducros sensor the sweep also computes it for its
 // cells and stores it for the y and z sweeps.
 //
-// Bound by the vector units (0.88 busy in FP64), so by the lanes that hold no
-// face.  Row tiles of one wave, 64 less the halo's SW - 1, spent 192 lanes on a
+// Bound by the vector units and, on large grids, by memory as well (FP64 SLAU6 NS
+// 256^3: units busy 0.58 to 0.61 of the time, 4.4 TB/s), so by the lanes that hold
+// no face.  Row tiles of one wave, 64 less the halo's SW - 1, spent 192 lanes on a
 // row of 124 cells and 128 on one of 80; runs lose one lane in 64, the halo cells'
 // loads and the end of a band.  Measured (us), tiles -> runs: FP64 SLAU6 NS 80 x
 // 112 x 48 38 -> 29, 124^3 122 -> 101, 192^3 417 -> 366; Hybrid6 LES 64^3 35 -> 26,
@@ -903,13 +904,13 @@ __global__ __launch_bounds__(256) void k_sweep_x(SweepArgs<R, S> a) {
 // and one face per lane (its cell's left face), and the halo positions of the
 // LDS row hold the periodic images of the row's other end.  The face left of
 // the first cell is then the face right of the last: its window cells are the
-// periodic images of that face's window cells.  The run computes the same face from the ghost cells, which hold exact copies of those images
-// once a z-sweep epilogue has written the primitive set, so both give the
-// same bits.  Used for such primitive sets only (k_prim takes the ghost
-// layers of an uploaded state as they are), on fully periodic grids, without
-// LES (the ghost SGS fields are copies of the layer next to
-// the boundary), and not for ORDER 2 with the
-// sensor, whose ghost cells copy the adjacent interior sensor
+// periodic images of that face's window cells.  The run computes the same face
+// from the ghost cells, which hold exact copies of those images once a z-sweep
+// epilogue has written the primitive set, so both give the same bits.  Used for
+// such primitive sets only (k_prim takes the ghost layers of an uploaded state as
+// they are), on fully periodic grids, without LES (the ghost SGS fields are copies
+// of the layer next to the boundary), and not for ORDER 2 with the sensor, whose
+// ghost cells copy the adjacent interior sensor
 // (calc_hybrid.f90:54-71) instead of the image's.
 // ---------------------------------------------------------------------------
 template <int ORDER, int SCHEME, int VISC>
@@ -1168,7 +1169,11 @@ inline int even_lseg(int cells, int lseg) {
 // 32^3 to 256^3, KEEP4 and SLAU6, Euler and NS, both precisions: on average
 // 3%, at most 19%, above the best length found by trying all; always 64 cells
 // took 100 us for a KEEP4 NS y sweep at 64^3 (16 workgroups), this rule's 4
-// cells 16 us; at 256^3 both lie within 2%.
+// cells 16 us.  At 256^3, where it gives 43 cells, both lie within 6%: FP64 SLAU6
+// NS y 658 us and 666, z 1025 and 1043; KEEP4 NS y 488 and 518, z 955 and 947; FP32
+// SLAU6 NS y 343 and 358, z 728 and 742.  The y and the z sweep share the two
+// constants although their best lengths differ: KEEP4 NS z takes 838 us in segments
+// of 256.
 inline int pick_lseg(const LineWork* p, int n, int occ, int cus) {
   int longest = 1;
   for (int m = 0; m < n; ++m) longest = std::max(longest, p[m].cells);
@@ -1199,8 +1204,8 @@ inline int pick_lseg(const LineWork* p, int n, int occ, int cus) {
 // face.  That and loading a face's operands after its convective half (below)
 // let the SLAU6 NS sweeps run two waves per SIMD (254 and 256 registers; with
 // the whole window in registers 368 and 416, one wave) on 74 KB of LDS per
-// workgroup, with 13% fewer vector instructions.  The sweeps are bound by the
-// vector units (y, 0.73 busy) and by memory (z).  Best segment length on either
+// workgroup, with 13% fewer vector instructions.  At 256^3 y is bound by the vector
+// units and latency (units busy 0.56 to 0.60 of the time), z by memory.  Best segment length on either
 // side: at 256^3 y 764 -> 700, z 1091 -> 1036 us; at 192^3 y 425 -> 355, z 538 ->
 // 461 us; KEEP4 NS at 64^3 y 18 -> 16, z 23 -> 21 us.  FP32 windows fit two to
 // four waves as they are, and their ring was slower (SLAU6 NS at 128^3: y 58 ->
@@ -1294,21 +1299,18 @@ __device__ __forceinline__ void sweep_line_tile(const SweepArgs<R, S>& a, int bx
     if constexpr (RING) ring_put<ORDER, SCHEME, VISC, VO>(mine + m * 256, win[m]);
   }
   int head = 0;  // ring slot of the window's first cell
-  // Software pipeline: the values of the cell that enters the window at face
-  // f+1, and the residual (and state) of the cell that face f+1 completes,
-  // are loaded while face f is computed, so that one face's arithmetic
-  // covers the memory latency of the next.
-  RC nxt;
+  RC nxt;  // the raw values of the cell that enters the window next
   {
     const int sp = s0 - 1 + St::HW;
     fetch_cell<S, DIR, ORDER, SCHEME, VISC, VO>(P, g, mbase + sp * stride, mbase + wrap(sp) * stride, nxt);
   }
   R Fp[5];
   CellState<DIR, EP> cs;
-  // Software pipeline.  The values of the cell that enters the window at face
-  // f+1 are loaded while face f is computed.  Windows held in registers through
-  // a viscous face issue its transverse stencils, and the state of the cell that
-  // face f+1 completes, a whole face ahead.  With the ring the state of cell f,
+  // Software pipeline: the values of the cell that enters the window at face
+  // f+1 are loaded while face f is computed, so that one face's arithmetic covers
+  // the memory latency of the next.  Windows held in registers through a viscous
+  // face issue its transverse stencils, and the state of the cell that face f+1
+  // completes, a whole face ahead.  With the ring the state of cell f,
   // which face f completes, and the next cell's stencils are issued between the
   // two halves of face f, so that those registers are free during the convective
   // half; Euler sweeps load the state of cell f at the top of the iteration.

@@ -27,12 +27,15 @@ __device__ __forceinline__ unsigned launch_block() { return blockIdx.x + gridDim
 // z 1042 -> 1065; FP32 SLAU6 Euler 256^3 x 296 -> 270; FP32 Roe4 NS 190 x 187 x 181,
 // undivided before, y 145 -> 137, z 271 -> 253; six FP32 requests 138.9 -> 133.9 ms; over
 // the 256^3 Taylor-Green runs the step is the same within 0.6%.
-// Chunks of 16 are equal, of 8 and 64 a little slower.)  `few`: a launch of up to
-// 2048 workgroups, which the chip holds at once, is one run per XCD instead; the
-// line sweeps of a lone case take it (FP32 96^3 y, SLAU6 Euler 25.6 -> 24.7 us,
-// KEEP4 NS 17.7 -> 16.9), the x sweep and batches are faster in chunks (FP32 SLAU6
-// Euler 64^3 x 11.4 -> 10.4; the six requests 136.3 -> 133.9 ms).
-// The map is a permutation of [0, n).
+// Chunks of 16 are equal, of 8 and 64 a little slower.  The price is traffic beyond
+// L2: the x sweep's neighbours in z always come from another XCD's chunk.)  `few`: a
+// launch of up to 2048 workgroups is one run per XCD instead.  The 2-D stage needs it
+// (450 x 240, FP64: chunks 20.1 us, one run 14.1).  The line sweeps of a lone case
+// take it too, where the two differ by 5% at most, either way: FP32 SLAU6 Euler 96^3 y
+// with 864 workgroups chunks 22.9 us, one run 20.6; FP64 SLAU6 NS 160^3 z with 2400
+// chunks 309 us, one run 319, and with 1200 296 and 306.  The x sweep and batches
+// are faster in chunks (FP32 SLAU6 Euler 64^3 x 11.4 -> 10.4; the six requests 136.3
+// -> 133.9 ms).  The map is a permutation of [0, n).
 constexpr int XCD_CHUNK = 32;
 __device__ __forceinline__ int xcd_tile(int b, int n, bool few = false) {
   int base = 0, m = n;
