@@ -448,7 +448,8 @@ int ox_batch_admit_ic(ox_batch* b, const ox_config* cfg, const ox_ic* ic, int32_
  * replacing ox2d_set_state of a host array (2D_solver/OS/set.f90:28-46). */
 int ox2d_init_state(ox2d_solver* s);
 
-/* Page-locked host memory (hipHostMalloc): a device-to-host copy of a result
+/* Page-locked host memory (hipHostMalloc; a shared mapping of the driver's that
+ * a forked child does not have): a device-to-host copy of a result
  * into it runs at the host link's full rate, where a copy into pageable
  * memory is staged.  No counterpart in the reference; a serving helper for
  * callers of ox_batch_retire / ox_get_state that keep result buffers. */

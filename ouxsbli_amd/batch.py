@@ -118,7 +118,8 @@ class Batch:
     def __init__(self, hbm_budget: int, max_cases: int = 64, use_graph: bool = True, autotune: bool = True,
                  device: int = 0, pinned_results: bool = True):
         """``pinned_results``: retire() returns arrays on page-locked host
-        buffers from the process's pool (a faster device-to-host copy)."""
+        buffers from the process's pool (a faster device-to-host copy; a
+        forked child does not have such memory), else ordinary arrays."""
         self._lib = _native.load()
         c = _abi.OxBatchConfig()
         c.abi_version = _abi.OX_ABI_VERSION
